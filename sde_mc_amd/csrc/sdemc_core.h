@@ -1732,11 +1732,11 @@ __device__ __forceinline__ bool isclose32(float tau, float t) {
 // draws happen.
 template <int D, int FAM>
 struct AdaptRngSrc {
+  static constexpr bool SORTED = true;  // jump times never decrease
   NormalStream ns;
   JumpClock jc;  // the last jump drawn
   uint32_t plo, phi, k0, k1;
-  float tau1, J1, tau2, J2;
-  bool have2;
+  float tau1, J1, tau2, J2;  // tau2 < 0: no second jump drawn
   __device__ __forceinline__ void draw_next(const KModel& f, float& tau, float& J) {
     ++jc.j;
     jc.draw(k0, k1, plo, phi, f.inv_rate);
@@ -1752,9 +1752,8 @@ struct AdaptRngSrc {
     jc.init(k0, k1, plo, phi, f.rate, f.inv_rate);
     tau1 = jc.tau;
     J1 = f.rate > 0.0 ? jump_mark(f, jc.m1, jc.m2) : 0.0f;
-    tau2 = __builtin_inff();
+    tau2 = -1.0f;
     J2 = 0.0f;
-    have2 = false;
   }
   __device__ __forceinline__ float z(uint32_t row, int k) {
     constexpr int K = NK<D, FAM>::K;
@@ -1773,10 +1772,10 @@ struct AdaptRngSrc {
   __device__ __forceinline__ float next_time() const { return tau1; }
   __device__ __forceinline__ float mark(const KModel&) const { return J1; }
   __device__ __forceinline__ void advance(const KModel& f) {
-    if (have2) {
+    if (tau2 >= 0.0f) {
       tau1 = tau2;
       J1 = J2;
-      have2 = false;
+      tau2 = -1.0f;
     } else {
       draw_next(f, tau1, J1);
     }
@@ -1785,12 +1784,9 @@ struct AdaptRngSrc {
   // and whose pending jump falls before T (later ones are never used)
   __device__ __forceinline__ void refill(const KModel& f, bool lane_live, float T32) {
     if (f.rate > 0.0) {
-      const bool need = lane_live && !have2 && tau1 < T32;
+      const bool need = lane_live && tau2 < 0.0f && tau1 < T32;
       if (__any(need)) {
-        if (need) {
-          draw_next(f, tau2, J2);
-          have2 = true;
-        }
+        if (need) draw_next(f, tau2, J2);
       }
     }
   }
@@ -1798,6 +1794,7 @@ struct AdaptRngSrc {
 
 template <int D, int FAM>
 struct AdaptFixedSrc {
+  static constexpr bool SORTED = false;
   const sdemc_fixed_in* in;
   int64_t p, P;
   int32_t jn;
@@ -1832,21 +1829,87 @@ struct AdaptFixedSrc {
   __device__ __forceinline__ void refill(const KModel&, bool, float) {}
 };
 
+// min(a, b) of numbers (no NaN): the bare instruction, without the quieting
+// fminf adds to a scalar operand.
+__device__ __forceinline__ float min_num(float a, float b) {
+  float d;
+  asm("v_min_f32 %0, %1, %2" : "=v"(d) : "s"(a), "v"(b));
+  return d;
+}
+
+// The coefficient constants a step adds (a0, b0, c0) held in vector registers:
+// an instruction takes one scalar operand here, so fma(a1, x, a0) with both
+// constants scalar costs a register move of its own each time.
+template <int D, int FAM>
+struct HeldCoef {
+  float a0[D], b0[D], c0[D];
+  __device__ __forceinline__ void init(const KModel& f) {
+#pragma unroll
+    for (int i = 0; i < D; ++i) {
+      a0[i] = f.a0[i];
+      b0[i] = f.b0[i];
+      c0[i] = f.c0[i];
+      asm volatile("" : "+v"(a0[i]));
+      asm volatile("" : "+v"(b0[i]));
+      if (FAM == FAM_LEVY) asm volatile("" : "+v"(c0[i]));
+    }
+  }
+  // euler<D, FAM> with these constants (the families of the adapted grid)
+  __device__ __forceinline__ void step(const KModel& f, float (&x)[D], float dt,
+                                       const float (&dW)[D], const float (&dB)[D]) const {
+    if constexpr (FAM != FAM_MERTON && FAM != FAM_LEVY) {
+      euler<D, FAM>(f, x, dt, dW, dB);
+      return;
+    }
+    const float s0 = x[0];
+#pragma unroll
+    for (int i = 0; i < D; ++i) {
+      float a = __fmaf_rn(f.a1[i], x[i], a0[i]);
+      if (FAM == FAM_MERTON && i > 0) a = __fmaf_rn(f.ax[i], s0, a);
+      const float b = __fmaf_rn(f.b1[i], x[i], b0[i]);
+      const float t = __fmaf_rn(a, dt, x[i]);
+      if (FAM == FAM_MERTON) {
+        x[i] = __fmaf_rn(b, dW[i], t);
+      } else {
+        const float c = __fmaf_rn(f.c1[i], x[i], c0[i]);
+        x[i] = t + __fmaf_rn(c, dB[i], b * dW[i]);
+      }
+    }
+  }
+};
+
 // Single level on the adapted grid.  Returns the number of steps taken;
 // `overflow` is set when max_steps was reached before T.
+//
+// A row's clock is kept to two operations and one compare.  The step
+// dt = min(h, T - t, tau - t) is min(h, lim - t) with lim = min(tau, T): fp32
+// subtraction is monotone, and a nominal step cut at T stays cut at every later
+// row, so this is the reference's running h (solvers.py:187-191) bit for bit;
+// caller-supplied jump times need not be sorted and keep the running form.
+// A row ends in an event -- a jump, the horizon, the step limit -- only if t
+// reaches ev = min(tau - margin, T), margin above the tolerance of the jump
+// test; lim and ev change only in events.  A finished lane keeps its state in
+// xT and steps by zero, so no row needs a lane mask: the wavefront tests for
+// an event with one compare and branch.
 template <int D, int FAM, bool STORE, class SRC>
 __device__ int32_t path_adapted(const KJob& j, SRC& src, bool lane_valid, int64_t p,
                                 float (&x)[D], int& overflow, const StoreCtx& st) {
   constexpr int K = NK<D, FAM>::K;
   const KModel& f = j.m;
   const float T32 = (float)j.T;
+  const float margin = 2e-5f * T32 + 1e-11f;  // isclose32 allows 1e-12 + 1e-5 t, t <= T
   const int32_t max_steps = j.max_steps;
+  HeldCoef<D, FAM> co;
+  co.init(f);
   float h = j.h;
   float t = 0.0f;
+  float xT[D];
 #pragma unroll
-  for (int i = 0; i < D; ++i) x[i] = f.x0[i];
+  for (int i = 0; i < D; ++i) x[i] = xT[i] = f.x0[i];
   float tau = lane_valid ? src.next_time() : 0.0f;
   bool active = lane_valid && (t < T32);
+  float lim = active ? fminf(tau, T32) : t;
+  float ev = active ? fminf(tau - margin, T32) : __builtin_inff();
   int32_t steps = 0;
   overflow = 0;
   if (STORE && lane_valid) {
@@ -1867,86 +1930,108 @@ __device__ int32_t path_adapted(const KJob& j, SRC& src, bool lane_valid, int64_
   // step.
   constexpr int G = group_steps(K);
   const uint32_t refill_mask = (uint32_t)j.clock_win - 1u;
-  for (uint32_t row0 = 0; __any(active); row0 += G) {
-    if ((row0 & refill_mask) < (uint32_t)G) src.refill(f, active, T32);
+  uint64_t live = __ballot(active);
+  for (int32_t row0 = 0; live != 0; row0 += G) {
+    if (((uint32_t)row0 & refill_mask) < (uint32_t)G) src.refill(f, active, T32);
+    // the group in which max_steps falls: every row of it is looked at
+    const bool last = row0 + G >= max_steps;
+    if (last && active) ev = -__builtin_inff();
     float zq[G * K];
-    src.rows(row0, active, zq);
+    src.rows((uint32_t)row0, active, zq);
 #pragma unroll
     for (int q = 0; q < G; ++q) {
-      if (active && steps >= max_steps) {
-        overflow = 1;
-        active = false;
-      }
-      if (active) {
-        float dt, tn;
-        {
+      const int32_t row = row0 + q;  // rows taken so far by every live lane
+      float dt;
+      {
 #pragma clang fp contract(off)
+        if constexpr (SRC::SORTED) {
+          dt = min_num(h, lim - t);
+        } else {
           h = fminf(h, fmaxf(T32 - t, 0.0f));
-          dt = fminf(h, tau - t);
+          dt = fminf(h, lim - t);
         }
-        const float sq = __builtin_amdgcn_sqrtf(dt);
-        float zz[K];
+      }
+      const float sq = __builtin_amdgcn_sqrtf(dt);
+      float zz[K];
 #pragma unroll
-        for (int k = 0; k < K; ++k) zz[k] = zq[q * K + k];
-        float dW[D], dB[D], xo[D];
-        correlate<D, FAM>(f, zz, sq, dW, dB);
+      for (int k = 0; k < K; ++k) zz[k] = zq[q * K + k];
+      float dW[D], dB[D], xo[D];
+      correlate<D, FAM>(f, zz, sq, dW, dB);
 #pragma unroll
-        for (int i = 0; i < D; ++i) xo[i] = x[i];
-        euler<D, FAM>(f, x, dt, dW, dB);
-        {
+      for (int i = 0; i < D; ++i) xo[i] = x[i];
+      co.step(f, x, dt, dW, dB);
+      {
 #pragma clang fp contract(off)
-          tn = t + dt;
+        t = t + dt;
+      }
+      if (STORE && active) {
+        const int64_t r = (int64_t)(row + 1) * D;
+        if (st.left) {
+#pragma unroll
+          for (int i = 0; i < D; ++i) st.left[(r + i) * st.P + p] = x[i];
         }
-        t = tn;
-        ++steps;
-        if (STORE) {
-          const int64_t r = (int64_t)steps * D;
-          if (st.left) {
+        if (st.times) st.times[(int64_t)(row + 1) * st.P + p] = t;
+        if (st.normals) {
+          const int64_t rn = (int64_t)row * D * (DiagNoise<FAM>::value ? 1 : 2);
+          if (DiagNoise<FAM>::value) {
 #pragma unroll
-            for (int i = 0; i < D; ++i) st.left[(r + i) * st.P + p] = x[i];
-          }
-          if (st.times) st.times[(int64_t)steps * st.P + p] = t;
-          if (st.normals) {
-            const int64_t rn = (int64_t)(steps - 1) * D * (DiagNoise<FAM>::value ? 1 : 2);
-            if (DiagNoise<FAM>::value) {
+            for (int i = 0; i < D; ++i) st.normals[(rn + i) * st.P + p] = dW[i];
+          } else {
 #pragma unroll
-              for (int i = 0; i < D; ++i) st.normals[(rn + i) * st.P + p] = dW[i];
-            } else {
-#pragma unroll
-              for (int i = 0; i < D; ++i) {
-                st.normals[(rn + 2 * i) * st.P + p] = dW[i];
-                st.normals[(rn + 2 * i + 1) * st.P + p] = dB[i];
-              }
+            for (int i = 0; i < D; ++i) {
+              st.normals[(rn + 2 * i) * st.P + p] = dW[i];
+              st.normals[(rn + 2 * i + 1) * st.P + p] = dB[i];
             }
           }
         }
-        float Jap = 0.0f;
-        if (isclose32(tau, t)) {
-          const float J = src.mark(f);
-          if (f.exact) {
-            float y[D];
-#pragma unroll
-            for (int i = 0; i < D; ++i) y[i] = x[i];
-            add_jump(f, x, y, J);
-          } else {
-            add_jump(f, x, xo, J);
-          }
-          Jap = J;
-          src.advance(f);
-          tau = src.next_time();
-        }
-        if (STORE) {
-          const int64_t r = (int64_t)steps * D;
-#pragma unroll
-          for (int i = 0; i < D; ++i) {
-            st.paths[(r + i) * st.P + p] = x[i];
-            if (st.jumps) st.jumps[(r + i) * st.P + p] = Jap;
-          }
-        }
-        active = t < T32;
       }
+      float Jap = 0.0f;
+      bool done = false;
+      if (__any(t >= ev)) {  // live lanes only: a finished lane's ev is +inf
+        if (t >= ev) {
+          if (isclose32(tau, t)) {
+            const float J = src.mark(f);
+            if (f.exact) {
+              float y[D];
+#pragma unroll
+              for (int i = 0; i < D; ++i) y[i] = x[i];
+              add_jump(f, x, y, J);
+            } else {
+              add_jump(f, x, xo, J);
+            }
+            Jap = J;
+            src.advance(f);
+            tau = src.next_time();
+            lim = fminf(tau, T32);
+            ev = last ? -__builtin_inff() : fminf(tau - margin, T32);
+          }
+          const bool stop = !(t < T32);
+          if (stop || row + 1 >= max_steps) {
+            overflow = stop ? 0 : 1;
+            done = true;
+            steps = row + 1;
+            lim = t;
+            ev = __builtin_inff();
+#pragma unroll
+            for (int i = 0; i < D; ++i) xT[i] = x[i];
+          }
+        }
+        live &= ~__ballot(done);
+      }
+      if (STORE && active) {
+        const int64_t r = (int64_t)(row + 1) * D;
+#pragma unroll
+        for (int i = 0; i < D; ++i) {
+          st.paths[(r + i) * st.P + p] = x[i];
+          if (st.jumps) st.jumps[(r + i) * st.P + p] = Jap;
+        }
+      }
+      if (STORE) active = active && !done;
     }
+    if (!STORE) active = ((live >> __lane_id()) & 1u) != 0;
   }
+#pragma unroll
+  for (int i = 0; i < D; ++i) x[i] = xT[i];
   if (STORE && lane_valid) {
     // rows past this path's end repeat its final state (a finished path
     // takes zero-length steps while others run, solvers.py:182-191)
