@@ -37,7 +37,7 @@ __device__ __forceinline__ void chunk_body(const KJob& job, int64_t chunk, doubl
       else
         path_uniform_rng_mode<D, FAM, false, U, MODE == 1>(job, c, valid, x, st);
     } else {
-      AdaptRngSrc<D, FAM> src;
+      AdaptQueueSrc<D, FAM> src;
       src.init(job.m, c);
       path_adapted<D, FAM, false>(job, src, valid, p, x, ovf, st);
     }
@@ -47,7 +47,7 @@ __device__ __forceinline__ void chunk_body(const KJob& job, int64_t chunk, doubl
     if (GRID == SDEMC_GRID_UNIFORM) {
       path_uniform_rng_coupled<D, FAM>(job, c, xf, xc);
     } else {
-      AdaptRngSrc<D, FAM> src;
+      AdaptQueueSrc<D, FAM> src;
       src.init(job.m, c);
       path_adapted_coupled<D, FAM>(job, src, valid, xf, xc, ovf);
     }

@@ -157,6 +157,18 @@ __device__ __forceinline__ float fast_ln(float v) {
   return 0.693147180559945309f * __builtin_amdgcn_logf(v);
 }
 
+// n / d correctly rounded for operands whose quotient and residuals need no
+// scaling (d within a few binades of 1, |n| <= d, n zero or not tiny): the
+// reciprocal refined once and the quotient twice, without the scaling and
+// special cases of __fdiv_rn; the same bits with three instructions fewer.
+__device__ __forceinline__ float div_rn_unscaled(float n, float d) {
+  float r = __builtin_amdgcn_rcpf(d);
+  r = __fmaf_rn(__fmaf_rn(-d, r, 1.0f), r, r);
+  float q = n * r;
+  q = __fmaf_rn(__fmaf_rn(-d, q, n), r, q);
+  return __fmaf_rn(__fmaf_rn(-d, q, n), r, q);
+}
+
 // ln u for u = (w | 1) 2^-32 in (0,1), in fp32 from correctly rounded
 // operations only (division, fma, multiply, add), so a CPU reproduces it bit
 // for bit: u = m 2^e with m in [sqrt(1/2), sqrt(2)), ln m = 2 atanh(s),
@@ -173,7 +185,7 @@ __device__ __forceinline__ float ln_unit(uint32_t w) {
   e = hi ? e + 1 : e;
   const float sn = m - 1.0f;
   const float sd = m + 1.0f;
-  const float sq = __fdiv_rn(sn, sd);
+  const float sq = div_rn_unscaled(sn, sd);
   const float s2 = sq * sq;
   float p = __fmaf_rn(s2, 0.222222222f, 0.285714286f);
   p = __fmaf_rn(s2, p, 0.4f);
@@ -258,7 +270,8 @@ struct KJob {
   // k+1 jumps iff its uniform word w < pois_T[k]; the first mark is the
   // offset of w within its count's interval (see poisson_count)
   int32_t pois_mode;
-  int32_t clock_win;  // steps per jump-queue fill window (uniform grid), per jump-slot refill (adapted)
+  int32_t clock_win;  // steps per jump-queue fill window (uniform grid), per jump-slot refill (adapted CV)
+  int32_t queue_win;  // adapted grid: rows per jump-queue fill window
   uint32_t pois_T[16];
   double pois_inv[16];  // reciprocal width of count c's interval at [c - 1]
   // Uniform-grid step form (uniform_step): UFORM_GENERIC, or the step's
@@ -412,6 +425,10 @@ inline void make_kjob(const sdemc_job& j, KJob& k) {
     int32_t w = uniform ? 512 : 128;
     while (w > 4 && per_step * (double)w > per_window) w >>= 1;
     k.clock_win = w;
+    // the adapted grid's queue: the same four jumps per path per window
+    w = 512;
+    while (w > 4 && per_step * (double)w > 4.0) w >>= 1;
+    k.queue_win = w;
   }
   for (int q = 0; q < 16; ++q) {
     k.pois_T[q] = 0;
@@ -473,21 +490,29 @@ inline bool job_pois_mode(const sdemc_job& j) {
 // Branch selection compares the fp32 uniform with fp32 thresholds, as the
 // reference's torch.where on fp32 tensors does.
 // All four branches share one logarithm (fast_pow is exp2 of e log2 b and
-// fast_ln is ln 2 log2 v), so the function is straight-line code: the lanes
-// of a wavefront that land in different branches cost one evaluation, and
-// every value is the one the branch would compute.
+// fast_ln is ln 2 log2 v) and one form a u + b of its argument, selected by
+// operand, so the function is straight-line code: the lanes of a wavefront
+// that land in different branches cost one evaluation and no jump, and every
+// value is the one the branch would compute.
 __device__ __forceinline__ float levy_icdf(const KModel& f, float y) {
   const bool t1 = y <= f.lv[0];
-  const bool t2 = !t1 && y < f.lv[1];
-  const bool t3 = !t1 && !t2 && y < f.lv[2];
-  const float arg = t1 ? f.lv[3] * y
-                       : (t2 ? __fmaf_rn(f.lv[5], y, f.lv[6])
-                             : (t3 ? __fmaf_rn(f.lv[7], y, f.lv[8]) : f.lv[9] * (1.0f - y)));
-  const float lg = __builtin_amdgcn_logf(arg);
+  const bool t2 = y < f.lv[1];  // meant after t1, t3 after t2
+  const bool t3 = y < f.lv[2];
+  float a = t3 ? f.lv[7] : f.lv[9];
+  float b = t3 ? f.lv[8] : 0.0f;
+  float u = t3 ? y : 1.0f - y;
+  a = t2 ? f.lv[5] : a;
+  b = t2 ? f.lv[6] : b;
+  u = t2 ? y : u;
+  a = t1 ? f.lv[3] : a;
+  b = t1 ? 0.0f : b;
+  u = t1 ? y : u;
+  const float lg = __builtin_amdgcn_logf(__fmaf_rn(a, u, b));
   const float pw = __builtin_amdgcn_exp2f(f.lv[10] * lg);
   const float ln = 0.693147180559945309f * lg;
-  return t1 ? __fmaf_rn(ln, f.lv[4], -1.0f)
-            : (t2 ? -pw : (t3 ? pw : __fmaf_rn(-f.lv[4], ln, 1.0f)));
+  const float tail = __fmaf_rn(t1 ? f.lv[4] : -f.lv[4], ln, t1 ? -1.0f : 1.0f);
+  const float body = t2 ? -pw : pw;
+  return !t1 && t3 ? body : tail;
 }
 
 // Jump mark from two Philox words.
@@ -1759,16 +1784,6 @@ struct AdaptRngSrc {
     constexpr int K = NK<D, FAM>::K;
     return ns.get(row * K + k);
   }
-  // normals of rows row0 .. row0 + G - 1 (G = group_steps(K), row0 a
-  // multiple of G): G K / 6 whole blocks, zq[s K + k] = z(row0 + s, k)
-  static constexpr int G = group_steps(NK<D, FAM>::K);
-  __device__ __forceinline__ void rows(uint32_t row0, bool, float (&zq)[G * NK<D, FAM>::K]) {
-    constexpr int K = NK<D, FAM>::K;
-    const uint32_t b0 = row0 * (uint32_t)K / (uint32_t)NORMALS_PER_BLOCK;
-#pragma unroll
-    for (int b = 0; b < G * K / NORMALS_PER_BLOCK; ++b)
-      normal_block(b0 + b, plo, phi, k0, k1, &zq[NORMALS_PER_BLOCK * b]);
-  }
   __device__ __forceinline__ float next_time() const { return tau1; }
   __device__ __forceinline__ float mark(const KModel&) const { return J1; }
   __device__ __forceinline__ void advance(const KModel& f) {
@@ -1787,6 +1802,109 @@ struct AdaptRngSrc {
       const bool need = lane_live && tau2 < 0.0f && tau1 < T32;
       if (__any(need)) {
         if (need) draw_next(f, tau2, J2);
+      }
+    }
+  }
+};
+
+// Philox source of the adapted grid with the coming jumps drawn ahead into the
+// wavefront's ClockLds queue (k holds the arrival times as float bits): slot
+// i mod CLOCK_JQ of a lane holds its jump number i, jumps head .. jc.j of it
+// are queued, and the pending jump (tau_head) always is.  fill(), called by
+// the whole wavefront at the start of a window, draws for every lane the jumps
+// up to the window's end and the one after, in passes in which all lanes that
+// need one draw at once; a lane that uses up a full queue inside a window
+// draws in place.  Each jump takes its own Philox block and the arrival times
+// accumulate in order, so the grid and the marks are those of a jump-by-jump
+// clock.  Two jump slots per lane in registers, refilled for the wavefront about
+// twice per jump, left a tenth of the jumps to be drawn by one lane alone; the
+// queue leaves almost none.
+template <int D, int FAM>
+struct AdaptQueueSrc {
+  static constexpr bool SORTED = true;  // jump times never decrease
+  JumpClock jc;                         // the last jump drawn
+  uint32_t plo, phi, k0, k1, lane;
+  uint32_t head;
+  ClockLds* cq;
+  __device__ __forceinline__ void put(const KModel& f) {
+    cq->k[jc.j % CLOCK_JQ][lane] = __float_as_int(jc.tau);
+    cq->J[jc.j % CLOCK_JQ][lane] = f.rate > 0.0 ? jump_mark(f, jc.m1, jc.m2) : 0.0f;
+  }
+  __device__ __forceinline__ void draw_next(const KModel& f) {
+    ++jc.j;
+    jc.draw(k0, k1, plo, phi, f.inv_rate);
+    put(f);
+  }
+  // the next two jumps, their blocks and marks side by side
+  __device__ __forceinline__ void draw_pair(const KModel& f) {
+#pragma clang fp contract(off)
+    const uint32_t i = jc.j + 1u, i2 = jc.j + 2u;
+    const U4 w = philox4x32_10(i, STREAM_JUMP, plo, phi, k0, k1);
+    const U4 v = philox4x32_10(i2, STREAM_JUMP, plo, phi, k0, k1);
+    const float gap = -ln_unit(w.x) * f.inv_rate;
+    const float gap2 = -ln_unit(v.x) * f.inv_rate;
+    const float J = jump_mark(f, w.y, w.z), J2 = jump_mark(f, v.y, v.z);
+    const float tau = jc.tau + gap;
+    jc.tau = tau + gap2;
+    jc.j = i2;
+    cq->k[i % CLOCK_JQ][lane] = __float_as_int(tau);
+    cq->J[i % CLOCK_JQ][lane] = J;
+    cq->k[i2 % CLOCK_JQ][lane] = __float_as_int(jc.tau);
+    cq->J[i2 % CLOCK_JQ][lane] = J2;
+  }
+  __device__ __forceinline__ void init(const KModel& f, const PathCtx& c) {
+    k0 = c.k0;
+    k1 = c.k1;
+    plo = (uint32_t)c.path;
+    phi = (uint32_t)(c.path >> 32);
+    lane = __lane_id();
+    cq = reinterpret_cast<ClockLds*>(&pois_lds());
+    head = 0;
+    if (f.rate > 0.0) {
+      jc.j = 0xffffffffu;  // none drawn
+      jc.tau = 0.0f;
+      draw_pair(f);
+    } else {
+      jc.j = 0;
+      jc.tau = __builtin_inff();
+      put(f);
+    }
+  }
+  // normals of rows row0 .. row0 + G - 1 (G = group_steps(K), row0 a
+  // multiple of G): G K / 6 whole blocks, zq[s K + k] normal k of row row0 + s
+  static constexpr int G = group_steps(NK<D, FAM>::K);
+  __device__ __forceinline__ void rows(uint32_t row0, bool, float (&zq)[G * NK<D, FAM>::K]) {
+    constexpr int K = NK<D, FAM>::K;
+    const uint32_t b0 = row0 * (uint32_t)K / (uint32_t)NORMALS_PER_BLOCK;
+#pragma unroll
+    for (int b = 0; b < G * K / NORMALS_PER_BLOCK; ++b)
+      normal_block(b0 + b, plo, phi, k0, k1, &zq[NORMALS_PER_BLOCK * b]);
+  }
+  __device__ __forceinline__ float next_time(bool = true) const {
+    return __int_as_float(cq->k[head % CLOCK_JQ][lane]);
+  }
+  __device__ __forceinline__ float mark(const KModel&, bool) const {
+    return cq->J[head % CLOCK_JQ][lane];
+  }
+  // past the pending jump where `hit`; next_time() is then the one after
+  __device__ __forceinline__ void advance(const KModel& f, bool hit) {
+    const bool dry = hit && head == jc.j;
+    if (__builtin_expect(__any(dry), 0)) {
+      if (dry) draw_next(f);
+    }
+    head += hit ? 1u : 0u;
+  }
+  // whole wavefront: the jumps of every live lane up to time `until`, and the
+  // one after, as far as its queue holds them
+  __device__ __forceinline__ void fill(const KModel& f, bool live, float until) {
+    if (f.rate > 0.0) {
+      // two at a time: the second draw hides behind the first, and one drawn
+      // past the window stays queued (drawn one by one, 1-D Merton at 20 jumps a
+      // path takes 3% more)
+      for (;;) {
+        const bool need = live && jc.tau < until && jc.j - head < (uint32_t)(CLOCK_JQ - 2);
+        if (!__any(need)) break;
+        if (need) draw_pair(f);
       }
     }
   }
@@ -1819,14 +1937,14 @@ struct AdaptFixedSrc {
 #pragma unroll
       for (int k = 0; k < K; ++k) zq[q * K + k] = live ? z(row0 + (uint32_t)q, k) : 0.0f;
   }
-  __device__ __forceinline__ float next_time() const {
-    return jn < in->max_jumps ? in->jump_time_dev[(int64_t)jn * P + p] : __builtin_inff();
+  __device__ __forceinline__ float next_time(bool hit = true) const {
+    return hit && jn < in->max_jumps ? in->jump_time_dev[(int64_t)jn * P + p] : __builtin_inff();
   }
-  __device__ __forceinline__ float mark(const KModel&) const {
-    return jn < in->max_jumps ? in->jump_size_dev[(int64_t)jn * P + p] : 0.0f;
+  __device__ __forceinline__ float mark(const KModel&, bool hit) const {
+    return hit && jn < in->max_jumps ? in->jump_size_dev[(int64_t)jn * P + p] : 0.0f;
   }
-  __device__ __forceinline__ void advance(const KModel&) { ++jn; }
-  __device__ __forceinline__ void refill(const KModel&, bool, float) {}
+  __device__ __forceinline__ void advance(const KModel&, bool hit) { jn += hit ? 1 : 0; }
+  __device__ __forceinline__ void fill(const KModel&, bool, float) {}
 };
 
 // min(a, b) of numbers (no NaN): the bare instruction, without the quieting
@@ -1924,15 +2042,16 @@ __device__ int32_t path_adapted(const KJob& j, SRC& src, bool lane_valid, int64_
   // every live lane is at row i: the normals of rows i .. i + G - 1 are drawn
   // for the wavefront together every G iterations (G = group_steps(K), whole
   // blocks), in the stream's layout (row r, normal k is index r K + k).  The
-  // second jump slots are refilled in the first group at or after every
-  // multiple of clock_win iterations (a power of two from 4: about half a
-  // jump per path between refills), a jump beyond them being drawn in the
-  // step.
+  // jump queue is filled every win rows, which advance a path by win h at most.
   constexpr int G = group_steps(K);
-  const uint32_t refill_mask = (uint32_t)j.clock_win - 1u;
+  const int32_t win = ((j.queue_win + G - 1) / G) * G;
+  int32_t wend = 0;
   uint64_t live = __ballot(active);
   for (int32_t row0 = 0; live != 0; row0 += G) {
-    if (((uint32_t)row0 & refill_mask) < (uint32_t)G) src.refill(f, active, T32);
+    if (row0 >= wend) {
+      wend = row0 + win;
+      src.fill(f, active, fminf(t + (float)win * j.h, T32));
+    }
     // the group in which max_steps falls: every row of it is looked at
     const bool last = row0 + G >= max_steps;
     if (last && active) ev = -__builtin_inff();
@@ -1988,25 +2107,25 @@ __device__ int32_t path_adapted(const KJob& j, SRC& src, bool lane_valid, int64_
       float Jap = 0.0f;
       bool done = false;
       if (__any(t >= ev)) {  // live lanes only: a finished lane's ev is +inf
-        if (t >= ev) {
-          if (isclose32(tau, t)) {
-            const float J = src.mark(f);
-            if (f.exact) {
-              float y[D];
+        // written so that the event's common course takes no branch: a taken
+        // one costs a wavefront that has its SIMD to itself about as long as
+        // ten instructions
+        if (t >= ev && isclose32(tau, t)) {
+          const float J = src.mark(f, true);
 #pragma unroll
-              for (int i = 0; i < D; ++i) y[i] = x[i];
-              add_jump(f, x, y, J);
-            } else {
-              add_jump(f, x, xo, J);
-            }
-            Jap = J;
-            src.advance(f);
-            tau = src.next_time();
-            lim = fminf(tau, T32);
-            ev = last ? -__builtin_inff() : fminf(tau - margin, T32);
+          for (int i = 0; i < D; ++i) {
+            const float y = f.exact ? x[i] : xo[i];  // add_jump
+            x[i] = __fmaf_rn(__fmaf_rn(f.j1[i], y, f.j0[i]), J, x[i]);
           }
+          Jap = J;
+          src.advance(f, true);
+          tau = src.next_time(true);
+          lim = fminf(tau, T32);
+          ev = last ? -__builtin_inff() : fminf(tau - margin, T32);
+        }
+        if (__builtin_expect(last || __any(t >= T32 && ev != __builtin_inff()), 0)) {
           const bool stop = !(t < T32);
-          if (stop || row + 1 >= max_steps) {
+          if (ev != __builtin_inff() && (stop || row + 1 >= max_steps)) {
             overflow = stop ? 0 : 1;
             done = true;
             steps = row + 1;
@@ -2015,8 +2134,8 @@ __device__ int32_t path_adapted(const KJob& j, SRC& src, bool lane_valid, int64_
 #pragma unroll
             for (int i = 0; i < D; ++i) xT[i] = x[i];
           }
+          live &= ~__ballot(done);
         }
-        live &= ~__ballot(done);
       }
       if (STORE && active) {
         const int64_t r = (int64_t)(row + 1) * D;
@@ -2051,11 +2170,15 @@ __device__ int32_t path_adapted(const KJob& j, SRC& src, bool lane_valid, int64_
 // Coupled pair on the adapted grid (solvers.py:228-307): per iteration M fine
 // sub-steps toward the pending jump time, then one coarse step driven by the
 // sum of the fine increments; a jump that falls now hits both levels, with
-// the fine coefficient taken before the last fine sub-step.
+// the fine coefficient taken before the last fine sub-step.  Every live lane is
+// at the same sub-step, so the sub-steps of all iterations run as one sequence
+// of rows whose normals are drawn G rows at a time in whole blocks
+// (path_adapted), the coarse half riding along every M rows.
 template <int D, int FAM, class SRC>
 __device__ int32_t path_adapted_coupled(const KJob& j, SRC& src, bool lane_valid,
                                         float (&xf)[D], float (&xc)[D], int& overflow) {
   constexpr int K = NK<D, FAM>::K;
+  constexpr int G = group_steps(K);
   const KModel& f = j.m;
   const int32_t M = j.M;
   const int32_t max_steps = j.max_steps;
@@ -2074,29 +2197,36 @@ __device__ int32_t path_adapted_coupled(const KJob& j, SRC& src, bool lane_valid
   }
   float tau = lane_valid ? src.next_time() : 0.0f;
   bool active = lane_valid && (tf < T32);
-  int32_t it = 0;
+  int32_t steps = 0;
   overflow = 0;
-  int32_t iter = 0;
-  int32_t refill_mask = j.clock_win - 1;  // a power of two minus one
-  while (refill_mask > 0 && (refill_mask + 1) * M > j.clock_win) refill_mask >>= 1;
-  while (__any(active)) {
-    // second jump slots for the wavefront together, every clock_win / M
-    // iterations (an iteration is M fine steps; the jumps keep their Philox
-    // blocks, so the marks are those drawn one by one)
-    if ((iter++ & refill_mask) == 0) src.refill(f, active, T32);
-    if (active && it >= max_steps) {
-      overflow = 1;
-      active = false;
-    }
-    if (active) {
-      float sW[D], sB[D], xfo[D];
+  int32_t it = 0;  // iterations taken by every live lane
+  int32_t cm = 0;  // fine sub-steps taken in the current iteration
+  float sW[D], sB[D], xfo[D];
 #pragma unroll
-      for (int i = 0; i < D; ++i) {
-        sW[i] = 0.0f;
-        sB[i] = 0.0f;
-        xfo[i] = xf[i];
+  for (int i = 0; i < D; ++i) {
+    sW[i] = 0.0f;
+    sB[i] = 0.0f;
+    xfo[i] = xf[i];
+  }
+  const int32_t win = ((j.queue_win + G - 1) / G) * G;
+  int32_t wend = 0;
+  for (int32_t row0 = 0; __any(active); row0 += G) {
+    if (row0 >= wend) {
+      wend = row0 + win;
+      src.fill(f, active, fminf(tf + (float)win * j.h, T32));
+    }
+    float zq[G * K];
+    src.rows((uint32_t)row0, active, zq);
+#pragma unroll
+    for (int q = 0; q < G; ++q) {
+      if (cm == 0 && it >= max_steps) {  // scalar: the live lanes run out together
+        if (active) {
+          overflow = 1;
+          steps = it;
+        }
+        active = false;
       }
-      for (int32_t s = 0; s < M; ++s) {
+      if (active) {
         float dt;
         {
 #pragma clang fp contract(off)
@@ -2106,7 +2236,7 @@ __device__ int32_t path_adapted_coupled(const KJob& j, SRC& src, bool lane_valid
         const float sq = __builtin_amdgcn_sqrtf(dt);
         float zz[K];
 #pragma unroll
-        for (int k = 0; k < K; ++k) zz[k] = src.z((uint32_t)(it * M + s), k);
+        for (int k = 0; k < K; ++k) zz[k] = zq[q * K + k];
         float dW[D], dB[D];
         correlate<D, FAM>(f, zz, sq, dW, dB);
 #pragma unroll
@@ -2122,42 +2252,56 @@ __device__ int32_t path_adapted_coupled(const KJob& j, SRC& src, bool lane_valid
           }
         }
       }
-      float dtc;
-      {
+      if (++cm == M) {
+        cm = 0;
+        ++it;
+        if (active) {
+          float dtc;
+          {
 #pragma clang fp contract(off)
-        hc = fminf(hc, fmaxf(T32 - tc, 0.0f));
-        dtc = fminf(hc, tau - tc);
-      }
-      float xco[D];
+            hc = fminf(hc, fmaxf(T32 - tc, 0.0f));
+            dtc = fminf(hc, tau - tc);
+          }
+          float xco[D];
 #pragma unroll
-      for (int i = 0; i < D; ++i) xco[i] = xc[i];
-      euler<D, FAM>(f, xc, dtc, sW, sB);
-      {
+          for (int i = 0; i < D; ++i) xco[i] = xc[i];
+          euler<D, FAM>(f, xc, dtc, sW, sB);
+          {
 #pragma clang fp contract(off)
-        tc = tc + dtc;
-      }
-      if (isclose32(tau, tf)) {
-        const float J = src.mark(f);
-        if (f.exact) {
-          float y[D];
+            tc = tc + dtc;
+          }
 #pragma unroll
-          for (int i = 0; i < D; ++i) y[i] = xf[i];
-          add_jump(f, xf, y, J);
+          for (int i = 0; i < D; ++i) {
+            sW[i] = 0.0f;
+            sB[i] = 0.0f;
+          }
+          const bool hit = isclose32(tau, tf);
+          if (hit) {
+            const float J = src.mark(f, true);
+            if (f.exact) {
+              float y[D];
 #pragma unroll
-          for (int i = 0; i < D; ++i) y[i] = xc[i];
-          add_jump(f, xc, y, J);
-        } else {
-          add_jump(f, xf, xfo, J);
-          add_jump(f, xc, xco, J);
+              for (int i = 0; i < D; ++i) y[i] = xf[i];
+              add_jump(f, xf, y, J);
+#pragma unroll
+              for (int i = 0; i < D; ++i) y[i] = xc[i];
+              add_jump(f, xc, y, J);
+            } else {
+              add_jump(f, xf, xfo, J);
+              add_jump(f, xc, xco, J);
+            }
+            src.advance(f, true);
+            tau = src.next_time();
+          }
+          if (!(tf < T32)) {
+            active = false;
+            steps = it;
+          }
         }
-        src.advance(f);
-        tau = src.next_time();
       }
-      ++it;
-      active = tf < T32;
     }
   }
-  return it;
+  return steps;
 }
 
 }  // namespace sdemc

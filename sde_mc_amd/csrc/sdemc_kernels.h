@@ -44,7 +44,7 @@ __global__ __launch_bounds__(512) void k_rng(const KJob job, double* __restrict_
     if (GRID == SDEMC_GRID_UNIFORM) {
       path_uniform_rng_mode<D, FAM, STORE, STORE ? 1 : 2, POIS>(job, c, valid, x, st);
     } else {
-      AdaptRngSrc<D, FAM> src;
+      AdaptQueueSrc<D, FAM> src;
       src.init(job.m, c);
       nsteps = path_adapted<D, FAM, STORE>(job, src, valid, p, x, ovf, st);
     }
@@ -60,7 +60,7 @@ __global__ __launch_bounds__(512) void k_rng(const KJob job, double* __restrict_
     if (GRID == SDEMC_GRID_UNIFORM) {
       path_uniform_rng_coupled<D, FAM>(job, c, xf, xc);
     } else {
-      AdaptRngSrc<D, FAM> src;
+      AdaptQueueSrc<D, FAM> src;
       src.init(job.m, c);
       nsteps = path_adapted_coupled<D, FAM>(job, src, valid, xf, xc, ovf);
     }
