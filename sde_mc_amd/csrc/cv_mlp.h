@@ -239,6 +239,8 @@ __global__ __launch_bounds__(256) void k_cv_uniform(const KJob job, const uint16
   for (int i = 0; i < D; ++i) x[i] = f.x0[i];
   const float h = job.h, sq = job.sqh;
   const int32_t n_cv = f_hidden > 0 ? cv_steps : 0;
+  CarriedStep<FAM> carried;
+  carried.init(f, h, f.x0[D - 1]);
   float cv = 0.0f;
   for (int32_t n = 0; n < job.steps; ++n) {
     float z[K], dW[D], dB[D];
@@ -252,7 +254,7 @@ __global__ __launch_bounds__(256) void k_cv_uniform(const KJob job, const uint16
       cv_mlp(0, f_hidden, lane, F, fo);
       cv = __fmaf_rn(fast_exp(-rate * t), cv_dot<D, FAM>(fo, dW, dB), cv);
     }
-    uniform_step<D, FAM>(job, x, z);
+    uniform_step<D, FAM>(job, x, z, carried);
   }
   float v = 0.0f;
   if (valid) {

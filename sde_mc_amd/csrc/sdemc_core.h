@@ -597,6 +597,17 @@ __device__ __forceinline__ float payoff_raw(const KPayoff& p, const float (&x)[D
   return v;
 }
 
+// sqrt(x) correctly rounded, x >= 2^-96 or 0: the hardware root (within one
+// unit) and its two neighbours, told apart by their exact residuals.
+__device__ __forceinline__ float sqrt_rn_unscaled(float x) {
+  float s = __builtin_amdgcn_sqrtf(x);
+  const float lo = __uint_as_float(__float_as_uint(s) - 1u);
+  const float hi = __uint_as_float(__float_as_uint(s) + 1u);
+  const float rl = __fmaf_rn(-lo, s, x), rh = __fmaf_rn(-hi, s, x);
+  s = rl <= 0.0f ? lo : s;
+  return rh > 0.0f ? hi : s;
+}
+
 // ---------------------------------------------------------------------------
 // Euler step (schemes.py:5-10) for one component and the jump update.
 // ---------------------------------------------------------------------------
@@ -610,13 +621,13 @@ __device__ __forceinline__ void euler(const KModel& f, float (&x)[D], float dt,
     static_assert(D == 2, "Heston state is (S, v)");
     const float S = x[0], v = x[1];
     const float a = f.a1[0] * S;
-    const float b = __fsqrt_rn(v) * S;
+    const float b = sqrt_rn_unscaled(v) * S;
     x[0] = __fmaf_rn(b, dW[0], __fmaf_rn(a, dt, S));
     const float A = __fmaf_rn(f.hv_kappa, dt, 1.0f);
     const float C = __fmaf_rn(f.hv_drift, dt, v);
     const float B = f.hv_xi * dW[1];
     const float disc = __fmaf_rn(B, B, 4.0f * A * C);
-    const float y = __fdiv_rn(B + __fsqrt_rn(disc), 2.0f * A);
+    const float y = __fdiv_rn(B + __builtin_amdgcn_sqrtf(disc), 2.0f * A);
     x[1] = y * y;
     return;
   }
@@ -647,6 +658,44 @@ __device__ __forceinline__ void euler(const KModel& f, float (&x)[D], float dt,
     }
   }
 }
+
+// The Heston step of a fixed step size, carrying sqrt(v): euler<2, FAM_HESTON>
+// bit for bit.  The new v is y^2 rounded, and the root of a rounded square is the
+// number itself, so the next step's sqrt(v) is y; the divisor 2 A is the same
+// every step, and with its correctly rounded reciprocal r one residual step
+// rounds n / (2 A) correctly (Markstein, IBM J. Res. Dev. 34, 1990): one root and
+// three operations for the quotient instead of two roots and a full division.
+// VALU-bound; 2^20 paths x 400 steps 772 -> 555 us, 10^4 paths 89 -> 72 us.
+struct HestonStep {
+  float sv, A4, den, r;
+  __device__ __forceinline__ void init(const KModel& f, float dt, float v) {
+    const float A = __fmaf_rn(f.hv_kappa, dt, 1.0f);
+    A4 = 4.0f * A;
+    den = 2.0f * A;
+    r = __fdiv_rn(1.0f, den);
+    sv = sqrt_rn_unscaled(v);
+  }
+  template <int D>
+  __device__ __forceinline__ void step(const KModel& f, float (&x)[D], float dt,
+                                       const float (&dW)[D]) {
+    static_assert(D == 2, "Heston state is (S, v)");
+    const float S = x[0];
+    const float a = f.a1[0] * S;
+    const float b = sv * S;
+    x[0] = __fmaf_rn(b, dW[0], __fmaf_rn(a, dt, S));
+    const float C = __fmaf_rn(f.hv_drift, dt, x[1]);
+    const float B = f.hv_xi * dW[1];
+    const float n = B + __builtin_amdgcn_sqrtf(__fmaf_rn(B, B, A4 * C));
+    const float q = n * r;
+    sv = __fmaf_rn(__fmaf_rn(-den, q, n), r, q);
+    x[1] = sv * sv;
+  }
+};
+struct NoStep {
+  __device__ __forceinline__ void init(const KModel&, float, float) {}
+};
+template <int FAM>
+using CarriedStep = std::conditional_t<FAM == FAM_HESTON, HestonStep, NoStep>;
 
 // x += g(y) * J with g(y) = j0 + j1 * y (sde.py:374-375, levy.py:119-120).
 template <int D>
@@ -754,7 +803,8 @@ __device__ __forceinline__ void correlate(const KModel& f, const float* z, float
 // the host.  Every kernel that steps a uniform grid from Philox normals
 // calls this, so their paths stay bit-identical.
 template <int D, int FAM>
-__device__ __forceinline__ void uniform_step(const KJob& j, float (&x)[D], const float* z) {
+__device__ __forceinline__ void uniform_step(const KJob& j, float (&x)[D], const float* z,
+                                             CarriedStep<FAM>& carried) {
   const KModel& f = j.m;
   if constexpr (FAM == FAM_MERTON || FAM == FAM_LEVY) {
     if (j.uform == UFORM_CONST) {
@@ -782,7 +832,8 @@ __device__ __forceinline__ void uniform_step(const KJob& j, float (&x)[D], const
   }
   float dW[D], dB[D];
   correlate<D, FAM>(f, z, j.sqh, dW, dB);
-  euler<D, FAM>(f, x, j.h, dW, dB);
+  if constexpr (FAM == FAM_HESTON) carried.step(f, x, j.h, dW);
+  else euler<D, FAM>(f, x, j.h, dW, dB);
 }
 
 // ---------------------------------------------------------------------------
@@ -1210,11 +1261,13 @@ struct CoarseAcc {
   }
   // the coarse step of size hc of the coarse state xc[0 .. D-1]
   template <int FAM>
-  __device__ __forceinline__ void step(const KModel& f, float hc, float* xc) {
+  __device__ __forceinline__ void step(const KModel& f, float hc, float* xc,
+                                       CarriedStep<FAM>& carried) {
     float y[D], yo[D];
 #pragma unroll
     for (int i = 0; i < D; ++i) y[i] = yo[i] = xc[i];
-    euler<D, FAM>(f, y, hc, sW, sB);
+    if constexpr (FAM == FAM_HESTON) carried.step(f, y, hc, sW);
+    else euler<D, FAM>(f, y, hc, sW, sB);
     if (f.exact) {
 #pragma unroll
       for (int i = 0; i < D; ++i) y[i] = __fmaf_rn(A[i], y[i], Bc[i]);
@@ -1283,6 +1336,9 @@ __device__ void path_uniform_rng_mode(const KJob& j, const PathCtx& c, bool lane
 #pragma unroll
     for (int i = 0; i < D; ++i) st.paths[(int64_t)i * st.P + c.p] = x[i];
   }
+  CarriedStep<FAM> fine, coarse;
+  fine.init(f, j.h, f.x0[D - 1]);
+  if constexpr (COUPLED) coarse.init(f, j.hc, f.x0[D - 1]);
   CoarseAcc<D> acc;
   int32_t cm = 0;  // fine steps taken in the current coarse step
   if constexpr (COUPLED) {
@@ -1351,7 +1407,7 @@ __device__ void path_uniform_rng_mode(const KJob& j, const PathCtx& c, bool lane
         if (COUPLED || (STORE && st.normals)) correlate<D, FAM>(f, &z[s * K], sq, dW, dB);
 #pragma unroll
         for (int i = 0; i < D; ++i) xo[i] = x[i];
-        uniform_step<D, FAM>(j, x, &z[s * K]);
+        uniform_step<D, FAM>(j, x, &z[s * K], fine);
         float jsum = 0.0f;
         if (!pois && n == hk) {
           do {
@@ -1424,7 +1480,7 @@ __device__ void path_uniform_rng_mode(const KJob& j, const PathCtx& c, bool lane
         if constexpr (COUPLED) {
           acc.increment(dW, dB);
           if (++cm == j.M) {
-            acc.template step<FAM>(f, j.hc, xc);
+            acc.template step<FAM>(f, j.hc, xc, coarse);
             acc.reset();
             cm = 0;
           }
