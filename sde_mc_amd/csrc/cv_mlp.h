@@ -31,6 +31,19 @@ typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 
 constexpr int CV_BLOCK_WORDS = 512;  // one operand fragment: 64 lanes x 8 bf16
+constexpr int CV_MAX_THREADS = 512;
+
+// Wavefronts per workgroup.  The workgroup's wavefronts share one LDS copy of
+// the weights (22 KB for a network of three hidden layers), so eight of them
+// leave room for the four wavefronts per SIMD that the registers allow where
+// workgroups of four with both networks fit three; a launch of fewer chunks
+// takes smaller workgroups, so that it reaches all 256 CUs.  2^18 Merton paths x
+// 300 adapted steps with an f and a g: 2782 -> 2613 us.
+inline int cv_waves_per_block(int64_t nchunks) {
+  int w = 8;
+  while (w > 1 && nchunks < 256 * (int64_t)w) w >>= 1;
+  return w;
+}
 
 __host__ __device__ constexpr int cv_blocks(int hidden) { return 8 * hidden - 2; }
 __host__ __device__ constexpr int cv_words(int hidden) {
@@ -216,7 +229,7 @@ __device__ __forceinline__ float cv_dot(const float (&fo)[8], const float (&dW)[
 // Uniform grid without jumps (apply_diffusion_control_variate): steps as in
 // path_uniform_rng, t_n = n h.
 template <int D, int FAM>
-__global__ __launch_bounds__(256) void k_cv_uniform(const KJob job, const uint16_t* fw,
+__global__ __launch_bounds__(CV_MAX_THREADS) void k_cv_uniform(const KJob job, const uint16_t* fw,
                                                     int32_t f_hidden, float rate,
                                                     int32_t cv_steps,
                                                     double* __restrict__ partials,
@@ -273,7 +286,7 @@ __global__ __launch_bounds__(256) void k_cv_uniform(const KJob job, const uint16
 // in lock-step across the wavefront so the products see all 64 lanes;
 // finished lanes ride along with their results masked.
 template <int D, int FAM>
-__global__ __launch_bounds__(256) void k_cv_adapted(const KJob job, const uint16_t* fw,
+__global__ __launch_bounds__(CV_MAX_THREADS) void k_cv_adapted(const KJob job, const uint16_t* fw,
                                                     int32_t f_hidden, const uint16_t* gw,
                                                     int32_t g_hidden, float rate, float comp,
                                                     int32_t cv_steps,
@@ -313,9 +326,9 @@ __global__ __launch_bounds__(256) void k_cv_adapted(const KJob job, const uint16
   int32_t steps = 0;
   int ovf = 0;
   float bcv = 0.0f, jcv = 0.0f, ccv = 0.0f;
-  int32_t iter = 0;
-  while (__any(row)) {
-    if ((iter++ & (job.clock_win - 1)) == 0) src.refill(f, active, T32);  // see path_adapted
+  // every live lane is at row `iter` (steps == iter)
+  for (int32_t iter = 0; __any(row); ++iter) {
+    if ((iter & (job.clock_win - 1)) == 0) src.refill(f, active, T32);
     if (active && steps >= max_steps) {
       ovf = 1;
       active = false;
@@ -351,7 +364,7 @@ __global__ __launch_bounds__(256) void k_cv_adapted(const KJob job, const uint16
         const float sq = __builtin_amdgcn_sqrtf(dt);
         float zz[K];
 #pragma unroll
-        for (int k = 0; k < K; ++k) zz[k] = src.z((uint32_t)steps, k);
+        for (int k = 0; k < K; ++k) zz[k] = src.z((uint32_t)iter, k);
         float dW[D], dB[D], xo[D];
         correlate<D, FAM>(f, zz, sq, dW, dB);
         if (use_f && steps < cv_steps) bcv = __fmaf_rn(disc, cv_dot<D, FAM>(fo, dW, dB), bcv);
@@ -411,14 +424,13 @@ struct CvLaunch {
   hipStream_t stream;
 };
 
-constexpr int CV_THREADS = 256;
-
 template <int D, int FAM>
 int launch_cv_uniform_d(const KJob& job, const CvLaunch& a, int64_t nchunks) {
-  const int64_t blocks = (nchunks + 3) / 4;
+  const int wpb = cv_waves_per_block(nchunks);
+  const int64_t blocks = (nchunks + wpb - 1) / wpb;
   if (blocks <= 0 || blocks > 0x7fffffffLL) return SDEMC_ERR_ARG;
   const size_t lds = (size_t)cv_words(a.f_hidden) * 2;
-  hipLaunchKernelGGL((k_cv_uniform<D, FAM>), dim3((unsigned)blocks), dim3(CV_THREADS), lds,
+  hipLaunchKernelGGL((k_cv_uniform<D, FAM>), dim3((unsigned)blocks), dim3(WAVE * wpb), lds,
                      a.stream, job, a.fw, a.f_hidden, a.rate, a.cv_steps, a.partials, a.cflags,
                      a.gamma, nchunks);
   return hipGetLastError() == hipSuccess ? SDEMC_OK : SDEMC_ERR_LAUNCH;
@@ -426,10 +438,11 @@ int launch_cv_uniform_d(const KJob& job, const CvLaunch& a, int64_t nchunks) {
 
 template <int D, int FAM>
 int launch_cv_adapted_d(const KJob& job, const CvLaunch& a, int64_t nchunks) {
-  const int64_t blocks = (nchunks + 3) / 4;
+  const int wpb = cv_waves_per_block(nchunks);
+  const int64_t blocks = (nchunks + wpb - 1) / wpb;
   if (blocks <= 0 || blocks > 0x7fffffffLL) return SDEMC_ERR_ARG;
   const size_t lds = (size_t)(cv_words(a.f_hidden) + cv_words(a.g_hidden)) * 2;
-  hipLaunchKernelGGL((k_cv_adapted<D, FAM>), dim3((unsigned)blocks), dim3(CV_THREADS), lds,
+  hipLaunchKernelGGL((k_cv_adapted<D, FAM>), dim3((unsigned)blocks), dim3(WAVE * wpb), lds,
                      a.stream, job, a.fw, a.f_hidden, a.gw, a.g_hidden, a.rate, a.comp,
                      a.cv_steps, a.partials, a.cflags, a.gamma, nchunks);
   return hipGetLastError() == hipSuccess ? SDEMC_OK : SDEMC_ERR_LAUNCH;
