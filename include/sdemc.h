@@ -334,6 +334,28 @@ typedef struct sdemc_cv_spec {
 /* bf16 words of a packed network with this many hidden layers. */
 size_t sdemc_cv_mlp_words(int32_t hidden_layers);
 
+/* One Linear layer of a network whose fp32 parameters are on the device:
+ * weight [out][in] row-major, bias [out] or null, and the eval-mode batch norms
+ * folded into it: `pre` on its inputs, `post` on its outputs (before the
+ * activation).  A batch norm is absent when var_dev is null; weight and bias
+ * are null when it has none. */
+typedef struct sdemc_cv_bn {
+  const float *weight_dev, *bias_dev, *mean_dev, *var_dev;
+  double eps;
+} sdemc_cv_bn;
+typedef struct sdemc_cv_layer {
+  const float *weight_dev, *bias_dev;
+  int32_t in, out;
+  sdemc_cv_bn pre, post;
+} sdemc_cv_layer;
+
+/* Pack a Linear (ReLU Linear)+ network on the device into the operand words
+ * above (words_dev: sdemc_cv_mlp_words(n_layers - 1) of them): n_layers Linear
+ * layers, hidden widths of at most 63, the first taking n_in (dim + 1) and
+ * the last giving n_out.  The parameters are read in stream order. */
+int sdemc_cv_pack(const sdemc_cv_layer* layers, int32_t n_layers, int32_t n_in, int32_t n_out,
+                  uint16_t* words_dev, void* stream);
+
 /* Control-variate run: stats_dev gets {sum, sum of squares, n, flags} of
  * gamma; gamma_dev (optional, [P] fp32) the per-path values. */
 int sdemc_cv_simulate(const sdemc_job* job, const sdemc_cv_spec* cv, double* stats_dev,

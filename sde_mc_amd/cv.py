@@ -37,44 +37,70 @@ class CvSpec(ctypes.Structure):
                 ("jump_comp", ctypes.c_double)]
 
 
-def _affine_layers(model):
-    """[(W, b)] of the network's Linear layers (fp64), eval-mode BatchNorm1d
-    folded in; checks the layer pattern Linear (ReLU Linear)*."""
+class CvBn(ctypes.Structure):
+    _fields_ = [("weight_dev", ctypes.c_void_p), ("bias_dev", ctypes.c_void_p),
+                ("mean_dev", ctypes.c_void_p), ("var_dev", ctypes.c_void_p),
+                ("eps", ctypes.c_double)]
+
+
+class CvLayer(ctypes.Structure):
+    _fields_ = [("weight_dev", ctypes.c_void_p), ("bias_dev", ctypes.c_void_p),
+                ("n_in", ctypes.c_int32), ("n_out", ctypes.c_int32), ("pre", CvBn), ("post", CvBn)]
+
+
+def layer_plan(model):
+    """[(linear, batch norm on its inputs or None, batch norms on its outputs)]
+    of a network, after checking the layer pattern Linear (ReLU Linear)+."""
     mods = [m for m in model.modules() if not isinstance(m, nn.Sequential) and m is not model
             and len(list(m.children())) == 0]
-    layers, pending_in, relus = [], None, []
+    layers, pending_in, relus = [], None, 0
     for m in mods:
         if isinstance(m, nn.BatchNorm1d):
             if m.training:
                 raise NotImplementedError('BatchNorm1d must be in eval mode to be folded')
-            s = (m.weight.detach().double() if m.affine else torch.ones(m.num_features, dtype=torch.float64))
-            s = s / torch.sqrt(m.running_var.double() + m.eps)
-            c = (m.bias.detach().double() if m.affine else 0.0) - s * m.running_mean.double()
-            if layers and len(relus) == len(layers) - 1:
-                W, b = layers[-1]                  # after a Linear: scale its outputs
-                layers[-1] = (s[:, None] * W, s * b + c)
-            else:                                   # on the inputs: fold into the next Linear
-                pending_in = (s, c)
+            if layers and relus == len(layers) - 1:
+                layers[-1][2].append(m)             # after a Linear: scales its outputs
+            else:
+                pending_in = m                      # on the inputs of the next Linear
         elif isinstance(m, nn.Linear):
-            W = m.weight.detach().double()
-            b = m.bias.detach().double() if m.bias is not None else torch.zeros(W.shape[0], dtype=torch.float64)
-            if pending_in is not None:
-                s, c = pending_in
-                b = b + W @ c
-                W = W * s[None, :]
-                pending_in = None
-            if len(relus) != len(layers):
+            if relus != len(layers):
                 raise NotImplementedError('Linear layers must be separated by ReLU')
-            layers.append((W, b))
+            layers.append((m, pending_in, []))
+            pending_in = None
         elif isinstance(m, nn.ReLU):
-            if len(relus) != len(layers) - 1:
+            if relus != len(layers) - 1:
                 raise NotImplementedError('one ReLU after each hidden Linear')
-            relus.append(m)
+            relus += 1
         else:
             raise NotImplementedError('%s has no device form' % type(m).__name__)
-    if len(layers) < 2 or len(relus) != len(layers) - 1:
+    if len(layers) < 2 or relus != len(layers) - 1:
         raise NotImplementedError('need Linear (ReLU Linear)+ with no final activation')
-    return [(W.cpu().numpy(), b.cpu().numpy()) for W, b in layers]
+    return layers
+
+
+def _bn_affine(m):
+    """(scale, shift) of an eval-mode BatchNorm1d, fp64."""
+    s = m.weight.detach().double() if m.affine else torch.ones_like(m.running_var, dtype=torch.float64)
+    s = s / torch.sqrt(m.running_var.double() + m.eps)
+    return s, (m.bias.detach().double() if m.affine else 0.0) - s * m.running_mean.double()
+
+
+def _affine_layers(model):
+    """[(W, b)] of the network's Linear layers (fp64, on the host), eval-mode
+    BatchNorm1d folded in."""
+    out = []
+    for lin, pre, post in layer_plan(model):
+        W = lin.weight.detach().double()
+        b = lin.bias.detach().double() if lin.bias is not None else W.new_zeros(W.shape[0])
+        if pre is not None:
+            s, c = _bn_affine(pre)
+            b = b + W @ c
+            W = W * s[None, :]
+        for m in post:
+            s, c = _bn_affine(m)
+            W, b = s[:, None] * W, s * b + c
+        out.append((W, b))
+    return [(W.cpu().numpy(), b.cpu().numpy()) for W, b in out]
 
 
 def _bf16_bits(a):
@@ -162,16 +188,77 @@ class ZeroNetwork:
     """Marker of the zero function (no work in the kernel)."""
 
 
+def _check_shape(plan, n_in, n_out):
+    """The limits of the packed form (padded_matrices)."""
+    if len(plan) - 1 > MAX_HIDDEN:
+        raise NotImplementedError('at most %d hidden layers' % MAX_HIDDEN)
+    if plan[0][0].in_features != n_in or plan[-1][0].out_features != n_out:
+        raise NotImplementedError('network must map R^%d to R^%d' % (n_in, n_out))
+    if n_in + 1 > 8 or n_out > MAX_OUT:
+        raise NotImplementedError('at most 7 inputs and %d outputs' % MAX_OUT)
+    if any(lin.out_features > HIDDEN_PAD - 1 for lin, _, _ in plan[:-1]):
+        raise NotImplementedError('hidden layers of at most %d units' % (HIDDEN_PAD - 1))
+
+
+def _device_layers(plan, device):
+    """The plan as sdemc_cv_layer entries when every parameter is an fp32
+    tensor on `device` that the packing kernel can read, else None (the host
+    packs then).  The second value holds the tensors the entries point into."""
+    held = []
+
+    def ptr(t):
+        if t is None:
+            return None
+        t = t.detach()
+        if t.dtype != torch.float32 or t.device != device or t.layout != torch.strided:
+            raise TypeError
+        held.append(t.contiguous())
+        return held[-1].data_ptr()
+
+    def bn(m):
+        e = CvBn()
+        if m is not None:
+            if m.running_var is None or m.running_mean is None:
+                raise TypeError
+            e.weight_dev, e.bias_dev = ptr(m.weight), ptr(m.bias)
+            e.mean_dev, e.var_dev, e.eps = ptr(m.running_mean), ptr(m.running_var), float(m.eps)
+        return e
+
+    entries = (CvLayer * len(plan))()
+    try:
+        for e, (lin, pre, post) in zip(entries, plan):
+            if len(post) > 1:
+                return None, None
+            e.weight_dev, e.bias_dev = ptr(lin.weight), ptr(lin.bias)
+            e.n_in, e.n_out = lin.in_features, lin.out_features
+            e.pre, e.post = bn(pre), bn(post[0] if post else None)
+    except TypeError:
+        return None, None
+    return entries, held
+
+
 class DeviceNetwork:
-    """A packed network resident on the device (None model: the zero function)."""
+    """A packed network resident on the device (None model: the zero function).
+    Networks whose parameters are on the device are packed there in one
+    launch (sdemc_cv_pack); the host packs any other."""
 
     def __init__(self, model, n_in, n_out, device):
         self.n_out = n_out
         if model is None or is_zero_network(model):
             self.hidden, self.words = 0, None
             return
-        arr, self.hidden = pack_network(model, n_in, n_out)
-        self.words = torch.from_numpy(arr.view(np.int16).copy()).to(device)
+        plan = layer_plan(model)
+        _check_shape(plan, n_in, n_out)
+        self.hidden = len(plan) - 1
+        entries, held = _device_layers(plan, device)
+        if entries is None:
+            arr, self.hidden = pack_network(model, n_in, n_out)
+            self.words = torch.from_numpy(arr.view(np.int16).copy()).to(device)
+            return
+        self.words = torch.empty(BLOCK * blocks(self.hidden), dtype=torch.int16, device=device)
+        L.check(L.lib().sdemc_cv_pack(entries, len(plan), n_in, n_out, E.ptr(self.words),
+                                      E.stream_ptr()), 'sdemc_cv_pack')
+        del held   # freed in stream order after the launch
 
     def c(self):
         m = CvMlp()

@@ -143,7 +143,7 @@ def _is_eval_packable(model):
     if getattr(model, 'sequential', False):
         return False
     try:
-        CV._affine_layers(model)
+        CV.layer_plan(model)
     except NotImplementedError:
         return False
     return True
