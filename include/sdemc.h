@@ -362,6 +362,21 @@ int sdemc_cv_simulate(const sdemc_job* job, const sdemc_cv_spec* cv, double* sta
                       float* gamma_dev, void* workspace_dev, size_t workspace_bytes,
                       void* stream);
 
+/* ---- training batches ---------------------------------------------------
+ * Gather the trajectories index[0 .. n_index) of up to SDEMC_GATHER_MAX fp32
+ * arrays, element (path, row, d) at src + path stride_path + row stride_row + d
+ * stride_dim, into contiguous [n_index][rows][dim] arrays.  An index outside
+ * [0, n_paths) reads nothing and gives NaN. */
+#define SDEMC_GATHER_MAX 8
+typedef struct sdemc_gather {
+  const float* src_dev;
+  float* dst_dev;
+  int64_t stride_path, stride_row, stride_dim;
+  int32_t rows, dim;
+} sdemc_gather;
+int sdemc_gather_paths(const sdemc_gather* arrays, int32_t n_arrays, const int64_t* index_dev,
+                       int64_t n_index, int64_t n_paths, void* stream);
+
 /* ---- batched persistent launch ------------------------------------------
  * A job table of max_jobs slots lives on the device in the library's own
  * prepared layout (sdemc_sizeof_prepared_job() bytes per slot), filled by

@@ -14,6 +14,7 @@ CHUNK = 64
 
 OK, ERR_ARG, ERR_UNSUPPORTED, ERR_LAUNCH, ERR_WORKSPACE, ERR_OVERFLOW, ERR_DEVICE = range(7)
 
+GATHER_MAX = 8
 ABI_VERSION = 5   # SDEMC_ABI_VERSION these structures follow
 # stats flag bits (enum sdemc_flag)
 FLAG_OVERFLOW, FLAG_JUMP_CSR, FLAG_CLASS, FLAG_TABLE = 1, 2, 4, 8
@@ -109,6 +110,12 @@ class SdemcError(RuntimeError):
         super().__init__(msg)
 
 
+class Gather(ctypes.Structure):
+    _fields_ = [("src_dev", ctypes.c_void_p), ("dst_dev", ctypes.c_void_p),
+                ("stride_path", ctypes.c_int64), ("stride_row", ctypes.c_int64),
+                ("stride_dim", ctypes.c_int64), ("rows", ctypes.c_int32), ("dim", ctypes.c_int32)]
+
+
 class HipUnavailableError(RuntimeError):
     """libsdemc.so is not built or no HIP device is present."""
 
@@ -148,6 +155,8 @@ _SIGS = {
     "sdemc_cv_simulate": (ctypes.c_int, [ctypes.POINTER(Job), ctypes.c_void_p, ctypes.c_void_p,
                                          ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t,
                                          ctypes.c_void_p]),
+    "sdemc_gather_paths": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int32, ctypes.c_void_p,
+                                          ctypes.c_int64, ctypes.c_int64, ctypes.c_void_p]),
     "sdemc_prepare_jobs": (ctypes.c_int, [ctypes.POINTER(Job), ctypes.c_int32,
                                           ctypes.POINTER(ctypes.c_int64), ctypes.c_void_p,
                                           ctypes.POINTER(ctypes.c_int32)]),

@@ -131,6 +131,52 @@ def simulate_fixed(job, fixed, device, out=None, stats=None):
     return stats
 
 
+def gather_paths(arrays, index):
+    """[a[index] for a in arrays], contiguous: the trajectories `index` (a list
+    of path indices) of stored arrays (paths, ...), gathered by one kernel
+    launch when they are fp32 on one HIP device with at most two axes after
+    the first that cannot be merged, else by torch."""
+    n = arrays[0].shape[0]
+    dev = arrays[0].device
+    one = dev.type == 'cuda' and len(arrays) <= L.GATHER_MAX and all(
+        type(a) is torch.Tensor and a.dtype == torch.float32 and a.device == dev
+        and a.shape[0] == n and a.dim() <= 4 and not a.requires_grad for a in arrays)
+    shapes = [_rows_and_dim(a) for a in arrays] if one else [None]
+    if any(s is None for s in shapes):
+        idx = torch.as_tensor(index, dtype=torch.int64, device=dev)
+        return [a[idx].contiguous() for a in arrays]
+    if len(index) and not (0 <= min(index) and max(index) < n):
+        raise IndexError('path index out of range')
+    idx = torch.tensor(index, dtype=torch.int64).to(dev)
+    out = [torch.empty((len(index),) + tuple(a.shape[1:]), dtype=torch.float32, device=dev)
+           for a in arrays]
+    g = (L.Gather * len(arrays))()
+    for e, a, o, (rows, dim, sr, sd) in zip(g, arrays, out, shapes):
+        e.src_dev, e.dst_dev = a.data_ptr(), o.data_ptr()
+        e.stride_path, e.stride_row, e.stride_dim = a.stride(0), sr, sd
+        e.rows, e.dim = rows, dim
+    with torch.cuda.device(dev):
+        L.check(L.lib().sdemc_gather_paths(g, len(arrays), ptr(idx), len(index), n, stream_ptr()),
+                'sdemc_gather_paths')
+    return out
+
+
+def _rows_and_dim(a):
+    """(rows, dim, row stride, dim stride) of a's axes after the first, merged
+    to two; None when they do not merge."""
+    axes = [(n, s) for n, s in zip(a.shape[1:], a.stride()[1:]) if n != 1]
+    merged = []
+    for n, s in axes:
+        if merged and merged[-1][1] == n * s:
+            merged[-1] = (merged[-1][0] * n, s)
+        else:
+            merged.append((n, s))
+    if len(merged) > 2:
+        return None
+    merged = [(1, 0)] * (2 - len(merged)) + merged
+    return merged[0][0], merged[1][0], merged[0][1], merged[1][1]
+
+
 def check_flags(flags, where):
     """Raise SdemcError for a statistics row whose flags word is not 0."""
     if flags != flags:  # NaN: no finalisation wrote this row

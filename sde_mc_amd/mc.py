@@ -15,13 +15,12 @@ import time
 
 import numpy as np
 import torch
-from torch.utils.data import DataLoader
 
 from . import _lib as L
 from . import cv as CV
 from . import engine as E
 from .helpers import ceil_mult, mc_estimates, remove_steps, sample_cov
-from .nets import AdaptedPathData, NormalPathData
+from .nets import AdaptedPathData, NormalPathData, PathLoader
 from .options import ConstantShortRate
 from .varred import (EarlyStopping, apply_adapted_control_variates,
                      apply_diffusion_control_variate, train_adapted_control_variates,
@@ -199,7 +198,7 @@ def simulate_data(trials, solver, payoff, discounter, bs=1000, inference=False):
     if inference:
         assert not trials % bs, 'Batch size should partition total trials evenly'
     paths, normals, payoffs = _store_paths(trials, solver, payoff, discounter)
-    return DataLoader(NormalPathData(paths, payoffs, normals), batch_size=int(bs),
+    return PathLoader(NormalPathData(paths, payoffs, normals), batch_size=int(bs),
                       shuffle=not inference, drop_last=not inference)
 
 
@@ -214,7 +213,7 @@ def simulate_adapted_data(trials, solver, payoff, discounter, bs=1000, inference
     ds = AdaptedPathData(paths[:, :total + 1], payoffs, normals[:, :total],
                          left_paths[:, :total + 1], time_paths[:, :total + 1],
                          jump_paths[:, :total + 1], total)
-    return DataLoader(ds, batch_size=int(bs), shuffle=not inference, drop_last=not inference)
+    return PathLoader(ds, batch_size=int(bs), shuffle=not inference, drop_last=not inference)
 
 
 def sim_train_control_variates(models, opt, solver, trials, payoff, discounter, sim_bs, bs,

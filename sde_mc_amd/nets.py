@@ -9,7 +9,9 @@ evaluated by torch on stored paths.
 import torch
 import torch.nn as nn
 import torch.optim as optim
-from torch.utils.data import Dataset
+from torch.utils.data import DataLoader, Dataset
+
+from . import engine as E
 
 
 class ControlVariate(nn.Module):
@@ -114,6 +116,11 @@ class NormalPathData(Dataset):
     def __getitem__(self, idx):
         return (self.paths[idx], self.normals[idx]), self.payoffs[idx]
 
+    def gather(self, index):
+        """The collated batch of these trajectories."""
+        *rows, payoffs = E.gather_paths([self.paths, self.normals, self.payoffs], index)
+        return [rows, payoffs]
+
 
 class NormalJumpsPathData(Dataset):
     """As NormalPathData with the jump marks (nets.py:178-189)."""
@@ -150,6 +157,25 @@ class AdaptedPathData(Dataset):
     def __getitem__(self, idx):
         return ((self.paths[idx], self.normals[idx], self.left_paths[idx], self.time_paths[idx],
                  self.jump_paths[idx]), self.payoffs[idx])
+
+    def gather(self, index):
+        """The collated batch of these trajectories."""
+        *rows, payoffs = E.gather_paths([self.paths, self.normals, self.left_paths,
+                                         self.time_paths, self.jump_paths, self.payoffs], index)
+        return [rows, payoffs]
+
+
+class PathLoader(DataLoader):
+    """DataLoader over a path dataset whose batches are gathered array by array
+    (dataset.gather) instead of being stacked from single trajectories: the
+    same batches in the same order (no workers)."""
+
+    def __iter__(self):
+        # a DataLoader takes its workers' base seed from the generator before
+        # the sampler takes its own: kept, so a seed gives the same shuffle
+        torch.empty((), dtype=torch.int64).random_(generator=self.generator)
+        for index in self.batch_sampler:
+            yield self.dataset.gather(index)
 
 
 def get_mlps(problem, num_layers, hidden_size, device):
