@@ -377,6 +377,17 @@ typedef struct sdemc_gather {
 int sdemc_gather_paths(const sdemc_gather* arrays, int32_t n_arrays, const int64_t* index_dev,
                        int64_t n_index, int64_t n_paths, void* stream);
 
+/* Parameter gradients of a Linear layer over `rows` points, fp32 throughout:
+ * dw [n_out][n_in] = dy^T x and (db non-null) db [n_out] = column sums of dy,
+ * for contiguous x [rows][n_in], dy [rows][n_out], rows >= 1, n_in <= 63,
+ * n_out <= 64.  workspace: sdemc_linear_grads_floats(...) fp32 values (0 for
+ * sizes outside the limits).  The order of summation depends only on the
+ * sizes. */
+size_t sdemc_linear_grads_floats(int64_t rows, int32_t n_in, int32_t n_out);
+int sdemc_linear_grads(const float* x_dev, const float* dy_dev, int64_t rows, int32_t n_in,
+                       int32_t n_out, float* dw_dev, float* db_dev, float* workspace_dev,
+                       size_t workspace_floats, void* stream);
+
 /* ---- batched persistent launch ------------------------------------------
  * A job table of max_jobs slots lives on the device in the library's own
  * prepared layout (sdemc_sizeof_prepared_job() bytes per slot), filled by

@@ -157,6 +157,12 @@ _SIGS = {
                                          ctypes.c_void_p]),
     "sdemc_gather_paths": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int32, ctypes.c_void_p,
                                           ctypes.c_int64, ctypes.c_int64, ctypes.c_void_p]),
+    "sdemc_linear_grads_floats": (ctypes.c_size_t, [ctypes.c_int64, ctypes.c_int32,
+                                                    ctypes.c_int32]),
+    "sdemc_linear_grads": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int64,
+                                          ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p,
+                                          ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t,
+                                          ctypes.c_void_p]),
     "sdemc_prepare_jobs": (ctypes.c_int, [ctypes.POINTER(Job), ctypes.c_int32,
                                           ctypes.POINTER(ctypes.c_int64), ctypes.c_void_p,
                                           ctypes.POINTER(ctypes.c_int32)]),

@@ -161,6 +161,21 @@ def gather_paths(arrays, index):
     return out
 
 
+def linear_grads(x, dy):
+    """(dy^T x, column sums of dy) of contiguous fp32 x (rows, n_in) and dy
+    (rows, n_out) on the current device (sdemc_linear_grads)."""
+    lib = L.lib()
+    rows, n_in = x.shape
+    n_out = dy.shape[1]
+    dw = torch.empty((n_out, n_in), dtype=torch.float32, device=x.device)
+    db = torch.empty(n_out, dtype=torch.float32, device=x.device)
+    ws = torch.empty(lib.sdemc_linear_grads_floats(rows, n_in, n_out), dtype=torch.float32,
+                     device=x.device)
+    L.check(lib.sdemc_linear_grads(ptr(x), ptr(dy), rows, n_in, n_out, ptr(dw), ptr(db), ptr(ws),
+                                   ws.numel(), stream_ptr()), 'sdemc_linear_grads')
+    return dw, db
+
+
 def _rows_and_dim(a):
     """(rows, dim, row stride, dim stride) of a's axes after the first, merged
     to two; None when they do not merge."""

@@ -18,7 +18,70 @@ import time
 import numpy as np
 import torch
 
+from . import engine as E
 from .helpers import partition, remove_steps
+from .nets import Mlp
+
+
+# Points per batch from which a layer's parameter gradients take the split
+# kernel.  Two gradients of a 50 x 50 layer: 16 us against the library's 25 at
+# 2048 points (launches in both), 16 against 95 at 16000, 16 against 128 at 48000
+# (1000 trajectories); smaller batches keep the module's own call.
+MIN_SPLIT_POINTS = 2048
+
+
+class _Linear(torch.autograd.Function):
+    """F.linear whose parameter gradients come from sdemc_linear_grads."""
+
+    @staticmethod
+    def forward(ctx, x, weight, bias):
+        ctx.save_for_backward(x, weight)
+        return torch.nn.functional.linear(x, weight, bias)
+
+    @staticmethod
+    def backward(ctx, dy):
+        x, weight = ctx.saved_tensors
+        dx = dw = db = None
+        if ctx.needs_input_grad[0]:
+            dx = dy @ weight
+        if ctx.needs_input_grad[1] or ctx.needs_input_grad[2]:
+            dw, db = E.linear_grads(x, dy.contiguous())
+        return dx, dw, db if ctx.needs_input_grad[2] else None
+
+
+def _plain_linear(m):
+    return (type(m) is torch.nn.Linear and m.weight.is_cuda and m.weight.dtype == torch.float32
+            and m.in_features <= 63 and m.out_features <= 64)
+
+
+def _training_forward(model):
+    """The model's forward as the training loops call it: the module itself,
+    or for an Mlp the same layers with _Linear for its fp32 Linear layers on
+    the device.  Only what a training step does passes through it (first-order
+    gradients of a plain module): a subclass, hooks, autocast or a
+    non-standard layer keep the module's own call."""
+    mods = [model, model.net] + list(model.net) if type(model) is Mlp else []
+    hooked = any(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks
+                 or m._backward_pre_hooks or 'forward' in m.__dict__ for m in mods) or any(
+        getattr(torch.nn.modules.module, '_global_%s_hooks' % k)
+        for k in ('forward', 'forward_pre', 'backward', 'backward_pre'))
+    if not mods or hooked or not any(_plain_linear(m) for m in mods) or \
+            type(model.net) is not torch.nn.Sequential:
+        return model
+
+    def forward(x):
+        if torch.is_autocast_enabled() or not (x.is_cuda and x.dtype == torch.float32
+                                               and x.dim() == 2 and len(x) >= MIN_SPLIT_POINTS):
+            return model(x)
+        for m in model.net:
+            if _plain_linear(m) and x.is_contiguous() and x.dtype == torch.float32:
+                x = _Linear.apply(x, m.weight, m.bias)
+            else:
+                x = m(x)
+        return x
+
+    forward.sequential = False
+    return forward
 
 
 class EarlyStopping:
@@ -103,10 +166,11 @@ def train_diffusion_control_variate(model, opt, dl, solver, discounter, epochs, 
     for epoch in range(epochs):
         t0 = time.time()
         model.train()
+        forward = _training_forward(model)
         total = 0.0
         for (paths, normals), payoffs in dl:
             opt.zero_grad()
-            loss = _diffusion_gammas(model, paths, normals, payoffs, time_points, discounts,
+            loss = _diffusion_gammas(forward, paths, normals, payoffs, time_points, discounts,
                                      solver, tol).var()
             total += loss.item()
             loss.backward()
@@ -173,10 +237,11 @@ def train_adapted_control_variates(models, opt, dl, solver, discounter, epochs=1
         t0 = time.time()
         for m in models:
             m.train()
+        forward = [_training_forward(m) for m in models]
         total = 0.0
         for batch, payoffs in dl:
             opt.zero_grad()
-            loss = _adapted_gammas(models, batch, payoffs, solver, discounter, tol).var()
+            loss = _adapted_gammas(forward, batch, payoffs, solver, discounter, tol).var()
             total += loss.item()
             loss.backward()
             opt.step()
