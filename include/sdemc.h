@@ -172,8 +172,9 @@ typedef struct sdemc_path_out {
                            its terminal state                                       */
   float* times_dev;     /* adapted only, [S+1][P] grid times                         */
   float* left_dev;      /* adapted only, [S+1][dim][P] pre-jump states              */
-  float* jumps_dev;     /* adapted only, [S+1][dim][P] applied jump marks           */
-  float* normals_dev;   /* [S][K][P] increments used (scaled and correlated);
+  float* jumps_dev;     /* [S+1][dim][P] applied jump marks, row 0 zero             */
+  float* normals_dev;   /* [S][K][P] increments used (scaled and correlated), zero
+                           past a path's end;
                            K = dim ('diag'), 2*dim ('indep': column-major pairs),
                            4 ('general': dW_0..3, zero beyond brown_dim)            */
 } sdemc_path_out;

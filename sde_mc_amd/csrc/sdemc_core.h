@@ -1334,7 +1334,10 @@ __device__ void path_uniform_rng_mode(const KJob& j, const PathCtx& c, bool lane
   for (int i = 0; i < D; ++i) x[i] = f.x0[i];
   if (STORE && lane_valid) {
 #pragma unroll
-    for (int i = 0; i < D; ++i) st.paths[(int64_t)i * st.P + c.p] = x[i];
+    for (int i = 0; i < D; ++i) {
+      st.paths[(int64_t)i * st.P + c.p] = x[i];
+      if (st.jumps) st.jumps[(int64_t)i * st.P + c.p] = 0.0f;
+    }
   }
   CarriedStep<FAM> fine, coarse;
   fine.init(f, j.h, f.x0[D - 1]);
@@ -2091,6 +2094,7 @@ __device__ int32_t path_adapted(const KJob& j, SRC& src, bool lane_valid, int64_
     for (int i = 0; i < D; ++i) {
       st.paths[(int64_t)i * st.P + p] = x[i];
       if (st.left) st.left[(int64_t)i * st.P + p] = x[i];
+      if (st.jumps) st.jumps[(int64_t)i * st.P + p] = 0.0f;
     }
     if (st.times) st.times[p] = 0.0f;
   }
@@ -2207,17 +2211,32 @@ __device__ int32_t path_adapted(const KJob& j, SRC& src, bool lane_valid, int64_
   }
 #pragma unroll
   for (int i = 0; i < D; ++i) x[i] = xT[i];
-  if (STORE && lane_valid) {
+  if (STORE) {
     // rows past this path's end repeat its final state (a finished path
-    // takes zero-length steps while others run, solvers.py:182-191)
-    for (int32_t r = steps + 1; r <= st.rows; ++r) {
+    // takes zero-length steps while others run, solvers.py:182-191) and take
+    // no increments; the wavefront walks the rows together, so a row's stores
+    // stay one line
+    int32_t from = steps;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+      const int32_t other = __shfl_xor(from, off);
+      from = other < from ? other : from;
+    }
+    constexpr int KN = D * (DiagNoise<FAM>::value ? 1 : 2);
+    for (int32_t r = from; r < st.rows; ++r) {
+      if (!lane_valid || r < steps) continue;
+      const int64_t q = (int64_t)(r + 1) * D;
 #pragma unroll
       for (int i = 0; i < D; ++i) {
-        st.paths[((int64_t)r * D + i) * st.P + p] = x[i];
-        if (st.left) st.left[((int64_t)r * D + i) * st.P + p] = x[i];
-        if (st.jumps) st.jumps[((int64_t)r * D + i) * st.P + p] = 0.0f;
+        st.paths[(q + i) * st.P + p] = x[i];
+        if (st.left) st.left[(q + i) * st.P + p] = x[i];
+        if (st.jumps) st.jumps[(q + i) * st.P + p] = 0.0f;
       }
-      if (st.times) st.times[(int64_t)r * st.P + p] = t;
+      if (st.times) st.times[(int64_t)(r + 1) * st.P + p] = t;
+      if (st.normals) {
+#pragma unroll
+        for (int k = 0; k < KN; ++k) st.normals[((int64_t)r * KN + k) * st.P + p] = 0.0f;
+      }
     }
   }
   return steps;

@@ -150,8 +150,9 @@ class SdeSolver(ABC):
             return nrm[:, :self.sde.brown_dim].permute(2, 0, 1)
         return nrm.reshape(nrm.shape[0], d, 2, nrm.shape[-1]).permute(3, 0, 1, 2)
 
-    def _materialise(self, bs, low_storage):
-        """One stored solve: paths [S+1][d][P] and the aux arrays, on device."""
+    def _materialise(self, bs, low_storage, jumps=True):
+        """One stored solve: paths [S+1][d][P] and the aux arrays, on device,
+        every element of them written by the kernel; `jumps`: store the marks."""
         dev = E.require_device()
         d = self.sde.dim
         job, _ = self.make_job(bs)
@@ -165,18 +166,25 @@ class SdeSolver(ABC):
         out.nsteps_dev = nsteps.data_ptr()
         aux = {}
         if not low_storage:
-            aux['normals'] = torch.zeros((rows, kn, bs), dtype=torch.float32, device=dev)
-            aux['jumps'] = torch.zeros((rows + 1, d, bs), dtype=torch.float32, device=dev)
+            aux['normals'] = torch.empty((rows, kn, bs), dtype=torch.float32, device=dev)
             out.normals_dev = aux['normals'].data_ptr()
-            out.jumps_dev = aux['jumps'].data_ptr()
+            if jumps:
+                aux['jumps'] = torch.empty((rows + 1, d, bs), dtype=torch.float32, device=dev)
+                out.jumps_dev = aux['jumps'].data_ptr()
             if adapted:
                 aux['times'] = torch.empty((rows + 1, bs), dtype=torch.float32, device=dev)
                 aux['left'] = torch.empty((rows + 1, d, bs), dtype=torch.float32, device=dev)
                 out.times_dev = aux['times'].data_ptr()
                 out.left_dev = aux['left'].data_ptr()
         stats = E.simulate(job, dev, out=out, wpb=self.waves_per_block)
+        total = job.steps
+        if adapted:
+            # the longest path's length comes back with the statistics
+            longest = nsteps.max().double().reshape(1) if bs > 0 else stats.new_zeros(1)
+            stats = torch.cat([stats, longest]).cpu()
+            total = int(stats[4])
         E.stats_to_host(stats, 'solve')
-        return job, rows, paths, nsteps, aux
+        return job, total, paths, aux
 
 
 class DiffusionSolver(SdeSolver):
@@ -185,7 +193,7 @@ class DiffusionSolver(SdeSolver):
     def solve(self, bs=1, return_normals=False):
         """paths (bs, N+1, dim) and the scaled correlated increments (solvers.py:68-88)."""
         bs = int(bs)
-        job, rows, paths, nsteps, aux = self._materialise(bs, low_storage=False)
+        _, _, paths, aux = self._materialise(bs, low_storage=False, jumps=False)
         od = self._out_device()
         p = paths.permute(2, 0, 1).to(od)
         return p, self._normals_out(aux['normals']).to(od)
@@ -233,14 +241,10 @@ class JumpDiffusionSolver(SdeSolver):
         """paths[:, :total_steps + 1] and (normals, time_paths, left_paths, total_steps,
         jump_paths) as in solvers.py:164-226 (aux is None under low_storage)."""
         bs = int(bs)
-        job, rows, paths, nsteps, aux = self._materialise(bs, low_storage)
+        job, total, paths, aux = self._materialise(bs, low_storage)
         od = self._out_device()
         d = self.sde.dim
         T = float(self.time_interval)
-        if job.grid == L.GRID_ADAPTED:
-            total = int(nsteps.max()) if bs > 0 else 0
-        else:
-            total = job.steps
         out_paths = paths[:total + 1].permute(2, 0, 1).to(od)
         if low_storage:
             return out_paths, (None, None, None, total, None)
