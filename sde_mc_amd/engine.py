@@ -7,7 +7,7 @@ import math
 
 import numpy as np
 import torch
-from scipy.stats import poisson
+from scipy.special import pdtr, pdtrik
 
 from . import _lib as L
 
@@ -28,24 +28,41 @@ def ptr(t):
     return ctypes.c_void_p(t.data_ptr()) if t is not None else ctypes.c_void_p(0)
 
 
+def poisson_quantile(q, mu):
+    """The q quantile of N ~ Poisson(mu), mu > 0: the real k at which the
+    distribution function, continued between the integers, takes the value q,
+    rounded up, and one less if that already reaches q.
+    (scipy.stats.poisson.ppf gives the same value in 50 us, half of the time of
+    building a job; this takes 3.)"""
+    k = math.ceil(float(pdtrik(q, mu)))
+    return k - 1 if k > 0 and pdtr(k - 1, mu) >= q else max(k, 0)
+
+
 def reference_max_jumps(rate, T):
     """The reference's storage bound on jumps per path (solvers.py:133)."""
     if rate <= 0:
         return 5
-    return max(int(T * poisson.ppf(1 - 1 / 1e9, rate)), 5)
+    return max(int(T * poisson_quantile(1 - 1 / 1e9, rate)), 5)
 
 
 def safe_max_jumps(rate, T):
     """A cap on jumps per path whose excess probability is below 1e-15."""
     if rate <= 0:
         return 8
-    return int(poisson.ppf(1 - 1e-15, rate * T)) + 16
+    return poisson_quantile(1 - 1e-15, rate * T) + 16
 
 
 def to_float(v):
     if torch.is_tensor(v):
-        return float(v.detach().double().cpu().reshape(-1)[0])
+        return float(v.item() if v.numel() == 1 else v.detach().reshape(-1)[0].item())
     return float(v)
+
+
+def total_rate(v):
+    """Sum of a jump rate given as a number or tensor, in fp64."""
+    if torch.is_tensor(v):
+        return float(v.item()) if v.numel() == 1 else float(v.double().sum())
+    return float(torch.as_tensor(v).double().sum())
 
 
 def fill_payoff(job, option, disc):

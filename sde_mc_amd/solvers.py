@@ -69,7 +69,7 @@ class SdeSolver(ABC):
         return L.GRID_ADAPTED if self.grid == 'adapted' else L.GRID_UNIFORM
 
     def _rate(self):
-        return float(torch.as_tensor(self.sde.jump_rate()).double().sum())
+        return E.total_rate(self.sde.jump_rate())
 
     def _take_paths(self, n):
         off = self.path_counter
