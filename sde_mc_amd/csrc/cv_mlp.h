@@ -267,7 +267,7 @@ __global__ __launch_bounds__(CV_MAX_THREADS) void k_cv_uniform(const KJob job, c
       cv_mlp(0, f_hidden, lane, F, fo);
       cv = __fmaf_rn(fast_exp(-rate * t), cv_dot<D, FAM>(fo, dW, dB), cv);
     }
-    uniform_step<D, FAM>(job, x, z, carried);
+    uniform_step<D, FAM>(job, x, z, carried, job.uA);
   }
   float v = 0.0f;
   if (valid) {

@@ -802,12 +802,24 @@ __device__ __forceinline__ void correlate(const KModel& f, const float* z, float
 // (schemes.py:5-10) with the products of the constant factors taken once on
 // the host.  Every kernel that steps a uniform grid from Philox normals
 // calls this, so their paths stay bit-identical.
-template <int D, int FAM>
+// UF: the job's form where the kernel is compiled for it (a form told apart in
+// every step takes five scalar branches a step), UFORM_ANY otherwise; uA: the
+// proportional form's constants, held in vector registers (see HeldCoef).
+constexpr int UFORM_ANY = -1;
+
+// The form most jobs of a family have, which its kernels are compiled for
+// beside the general loop.
+template <int FAM>
+constexpr int common_form() {
+  return FAM == FAM_MERTON ? (int)UFORM_PROP : (FAM == FAM_LEVY ? (int)UFORM_CONST : UFORM_ANY);
+}
+
+template <int D, int FAM, int UF = UFORM_ANY>
 __device__ __forceinline__ void uniform_step(const KJob& j, float (&x)[D], const float* z,
-                                             CarriedStep<FAM>& carried) {
+                                             CarriedStep<FAM>& carried, const float* uA) {
   const KModel& f = j.m;
   if constexpr (FAM == FAM_MERTON || FAM == FAM_LEVY) {
-    if (j.uform == UFORM_CONST) {
+    if (UF == UFORM_CONST || (UF == UFORM_ANY && j.uform == UFORM_CONST)) {
 #pragma unroll
       for (int i = 0; i < D; ++i) {
         float t = x[i] + j.uA[i];
@@ -818,10 +830,10 @@ __device__ __forceinline__ void uniform_step(const KJob& j, float (&x)[D], const
       }
       return;
     }
-    if (j.uform == UFORM_PROP) {
+    if (UF == UFORM_PROP || (UF == UFORM_ANY && j.uform == UFORM_PROP)) {
 #pragma unroll
       for (int i = 0; i < D; ++i) {
-        float g = __fmaf_rn(j.uW[i][0], z[0], j.uA[i]);
+        float g = __fmaf_rn(j.uW[i][0], z[0], uA[i]);
 #pragma unroll
         for (int q = 1; q <= i; ++q) g = __fmaf_rn(j.uW[i][q], z[q], g);
         if (FAM == FAM_LEVY) g = __fmaf_rn(j.uC[i], z[D], g);
@@ -973,12 +985,13 @@ struct PoisLds {
 
 // Arrival-clock jump queue of a wavefront (uniform grid): slot q of lane l
 // holds the step and the mark of the lane's q-th queued jump of the current
-// fill window, k = -1 past the last one.  It takes the space of PoisLds (a
+// fill window, k = -1 past the last one (a ninth slot is always -1, so a full
+// queue ends without a test).  It takes the space of PoisLds (a
 // kernel runs one jump mode); lane-contiguous, so every access is
 // conflict-free and each lane reads back only what it wrote itself.
 constexpr int CLOCK_JQ = 8;
 struct ClockLds {
-  int32_t k[CLOCK_JQ][WAVE];
+  int32_t k[CLOCK_JQ + 1][WAVE];
   float J[CLOCK_JQ][WAVE];
 };
 static_assert(sizeof(ClockLds) <= sizeof(PoisLds), "the clock queue shares the jump-list space");
@@ -1291,8 +1304,9 @@ struct CoarseAcc {
 // path_uniform_rng below dispatches on the job.
 // COUPLED: x is the fine path of an MLMC pair and xc (then non-null) its
 // coarse path, stepped every M = j.M fine steps by CoarseAcc.
-template <int D, int FAM, bool STORE, int U, bool POIS, bool COUPLED = false>
-__device__ void path_uniform_rng_mode(const KJob& j, const PathCtx& c, bool lane_valid,
+// UF: the step form the loop is compiled for (uniform_step).
+template <int D, int FAM, bool STORE, int U, bool POIS, bool COUPLED = false, int UF = UFORM_ANY>
+__device__ void path_uniform_rng_form(const KJob& j, const PathCtx& c, bool lane_valid,
                                       float (&x)[D], const StoreCtx& st,
                                       float* xc = nullptr) {
   constexpr int K = NK<D, FAM>::K;
@@ -1303,6 +1317,9 @@ __device__ void path_uniform_rng_mode(const KJob& j, const PathCtx& c, bool lane
   const float sq = j.sqh;
   const uint32_t plo = (uint32_t)c.path, phi = (uint32_t)(c.path >> 32);
   constexpr bool pois = POIS;
+  // the common forms' jump coefficients: the exponential Levy's are constant,
+  // the proportional ones are not (path_uniform_rng_mode asks for both)
+  const bool additive = UF == UFORM_CONST ? true : (UF == UFORM_PROP ? false : j.additive != 0);
   JumpClock jc;
   int32_t kj = 0x7fffffff;
   if (!pois) {
@@ -1339,6 +1356,12 @@ __device__ void path_uniform_rng_mode(const KJob& j, const PathCtx& c, bool lane
       if (st.jumps) st.jumps[(int64_t)i * st.P + c.p] = 0.0f;
     }
   }
+  float uA[D];
+#pragma unroll
+  for (int i = 0; i < D; ++i) {
+    uA[i] = j.uA[i];
+    if (UF == UFORM_PROP) asm volatile("" : "+v"(uA[i]));
+  }
   CarriedStep<FAM> fine, coarse;
   fine.init(f, j.h, f.x0[D - 1]);
   if constexpr (COUPLED) coarse.init(f, j.hc, f.x0[D - 1]);
@@ -1351,7 +1374,9 @@ __device__ void path_uniform_rng_mode(const KJob& j, const PathCtx& c, bool lane
   }
   uint32_t wjm = 0u;     // per-step Poisson mode: the lane's jumping steps of the window
   uint32_t wfirst = 0u;  // and its first item in the window's jump list
-  auto group = [&](int32_t n0, auto spill) {
+  // spill: some lane's jumps overflow its queue in this window; full: all G
+  // steps of the group lie on the grid
+  auto group = [&](int32_t n0, auto spill, auto full) {
     uint32_t jm = 0u;     // the lane's jumping steps of the group
     uint32_t first = 0u;  // its first item in the window's jump list
     if (pois) {
@@ -1404,18 +1429,20 @@ __device__ void path_uniform_rng_mode(const KJob& j, const PathCtx& c, bool lane
 #pragma unroll
     for (int s = 0; s < G; ++s) {
       const int32_t n = n0 + s;
-      if (n < N) {
+      if (decltype(full)::value || n < N) {
         float dW[D], dB[D], xo[D];
         // the increments themselves only for the coarse path and stored normals
         if (COUPLED || (STORE && st.normals)) correlate<D, FAM>(f, &z[s * K], sq, dW, dB);
 #pragma unroll
         for (int i = 0; i < D; ++i) xo[i] = x[i];
-        uniform_step<D, FAM>(j, x, &z[s * K], fine);
+        uniform_step<D, FAM, UF>(j, x, &z[s * K], fine, uA);
         float jsum = 0.0f;
-        if (!pois && n == hk) {
-          do {
+        // rare enough (and long) to be laid out of line: steps without a jump
+        // run straight on
+        if (!pois && __builtin_expect(__any(n == hk), 0)) {
+          while (n == hk) {
             const float J = cq->J[qh][lane];
-            if (j.additive) {  // fma(j1, y, j0) = j0 exactly: add_jump's bits, one operation
+            if (additive) {  // fma(j1, y, j0) = j0 exactly: add_jump's bits, one operation
 #pragma unroll
               for (int i = 0; i < D; ++i) x[i] = __fmaf_rn(f.j0[i], J, x[i]);
             } else if (f.exact) {
@@ -1429,10 +1456,10 @@ __device__ void path_uniform_rng_mode(const KJob& j, const PathCtx& c, bool lane
             jsum += J;
             if constexpr (COUPLED) acc.jump(f, J);
             ++qh;
-            hk = qh < CLOCK_JQ ? cq->k[qh][lane] : -1;
-          } while (n == hk);
+            hk = cq->k[qh][lane];
+          }
         }
-        if (pois && j.additive && ((jm >> s) & 1u)) {
+        if (pois && additive && ((jm >> s) & 1u)) {
           // constant jump coefficients: one total per jumping step
           const uint32_t it = first + (uint32_t)__builtin_popcount(jm & ((1u << s) - 1u));
           const float J = __uint_as_float(pl->v[it]);
@@ -1524,7 +1551,7 @@ __device__ void path_uniform_rng_mode(const KJob& j, const PathCtx& c, bool lane
   const int32_t win = ((j.clock_win + G * U - 1) / (G * U)) * (G * U);
   int32_t wend = 0;
   bool spill = false;
-  for (int32_t n0 = 0; n0 < N; n0 += G * U) {
+  auto window = [&](int32_t n0) {
     if (clock && n0 >= wend) {
       // the previous window's queue is used up: its jumps all fell before n0
       wend = n0 + win;
@@ -1540,23 +1567,49 @@ __device__ void path_uniform_rng_mode(const KJob& j, const PathCtx& c, bool lane
           tail = q + 1;
         }
       }
-      if (tail < CLOCK_JQ) cq->k[tail][lane] = -1;
+      cq->k[tail][lane] = -1;
       qh = 0;
       hk = cq->k[0][lane];
       spill = __any(kj < wend);
     }
+  };
+  int32_t n0 = 0;
+  for (; n0 + G * U <= N; n0 += G * U) {
+    window(n0);
     if (spill) {
-      group(n0, std::true_type{});
 #pragma unroll
-      for (int u = 1; u < U; ++u)
-        if (n0 + G * u < N) group(n0 + G * u, std::true_type{});
+      for (int u = 0; u < U; ++u) group(n0 + G * u, std::true_type{}, std::true_type{});
     } else {
-      group(n0, std::false_type{});
 #pragma unroll
-      for (int u = 1; u < U; ++u)
-        if (n0 + G * u < N) group(n0 + G * u, std::false_type{});
+      for (int u = 0; u < U; ++u) group(n0 + G * u, std::false_type{}, std::true_type{});
     }
   }
+  // the last steps of a grid that is no multiple of the stride
+  for (; n0 < N; n0 += G) {
+    window(n0);
+    group(n0, std::true_type{}, std::false_type{});
+  }
+}
+
+// The loop compiled for the family's common step form where the job has it
+// (storing kernels, bound by their writes, keep the general loop).  Told apart
+// in every step, the form, the end of the grid and the jump test were ten
+// scalar branches a step, which cost time even with eight wavefronts per SIMD:
+// 400 steps, 1-D GBM of 2^22 / 10^4 paths 954 -> 754 / 67 -> 33 us, 1-D Merton at
+// 2 jumps a path 1088 -> 831 / 85 -> 51 us, the 2-D Levy rainbow 3340 -> 2970 /
+// 199 -> 142 us.
+template <int D, int FAM, bool STORE, int U, bool POIS, bool COUPLED = false>
+__device__ __forceinline__ void path_uniform_rng_mode(const KJob& j, const PathCtx& c,
+                                                      bool lane_valid, float (&x)[D],
+                                                      const StoreCtx& st, float* xc = nullptr) {
+  constexpr int UF = STORE ? UFORM_ANY : common_form<FAM>();
+  if constexpr (UF != UFORM_ANY) {
+    if (j.uform == UF && (j.m.rate == 0.0 || (j.additive != 0) == (UF == UFORM_CONST))) {
+      path_uniform_rng_form<D, FAM, STORE, U, POIS, COUPLED, UF>(j, c, lane_valid, x, st, xc);
+      return;
+    }
+  }
+  path_uniform_rng_form<D, FAM, STORE, U, POIS, COUPLED>(j, c, lane_valid, x, st, xc);
 }
 
 template <int D, int FAM, bool STORE, int U = 1>
