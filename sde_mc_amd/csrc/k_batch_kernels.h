@@ -12,8 +12,8 @@ namespace sdemc {
 // One 64-path chunk of one job, RNG mode, no per-path outputs.  The result
 // equals the plain kernel's chunk: same Philox streams, same butterfly.
 // MODE: the uniform single-level path's jump mode, 0 the arrival clock, 1
-// per-step Poisson counts, -1 whichever the job has.
-template <int D, int FAM, int GRID, bool COUPLED, int U = 1, int MODE = -1>
+// per-step Poisson counts, -1 whichever the job has; UF: its step form.
+template <int D, int FAM, int GRID, bool COUPLED, int UF, int U = 1, int MODE = -1>
 __device__ __forceinline__ void chunk_body(const KJob& job, int64_t chunk, double* part,
                                            int32_t* cf) {
   const int lane = threadIdx.x & (WAVE - 1);
@@ -32,10 +32,10 @@ __device__ __forceinline__ void chunk_body(const KJob& job, int64_t chunk, doubl
   if (!COUPLED) {
     float x[D];
     if (GRID == SDEMC_GRID_UNIFORM) {
-      if constexpr (MODE < 0)
-        path_uniform_rng<D, FAM, false, U>(job, c, valid, x, st);
+      if (MODE == 1 || (MODE < 0 && job.pois_mode != 0))
+        path_uniform_rng_form<D, FAM, false, U, MODE != 0, false, UF>(job, c, valid, x, st);
       else
-        path_uniform_rng_mode<D, FAM, false, U, MODE == 1>(job, c, valid, x, st);
+        path_uniform_rng_form<D, FAM, false, U, MODE == 1, false, UF>(job, c, valid, x, st);
     } else {
       AdaptQueueSrc<D, FAM> src;
       src.init(job.m, c);
@@ -45,7 +45,8 @@ __device__ __forceinline__ void chunk_body(const KJob& job, int64_t chunk, doubl
   } else {
     float xf[D], xc[D];
     if (GRID == SDEMC_GRID_UNIFORM) {
-      path_uniform_rng_coupled<D, FAM>(job, c, xf, xc);
+      if (job.pois_mode != 0) path_uniform_rng_coupled<D, FAM, true, UF>(job, c, xf, xc);
+      else path_uniform_rng_coupled<D, FAM, false, UF>(job, c, xf, xc);
     } else {
       AdaptQueueSrc<D, FAM> src;
       src.init(job.m, c);
@@ -90,16 +91,29 @@ inline int32_t kjob_class_of(const KJob& k) {
 // The generic class calls each case's chunk body as a function of its own,
 // once per 64-path chunk: the cases are compiled one by one instead of all
 // inlined into one kernel body (about 1.5 minutes of compile time instead of
-// 15), and the call costs nothing next to a chunk's path work.
-template <int D, int FAM, int GRID, bool COUPLED>
+// 15), and the call costs nothing next to a chunk's path work.  The two step
+// forms of a uniform-grid case are functions of their own too.
+template <int D, int FAM, int GRID, bool COUPLED, int UF>
 __device__ __attribute__((noinline)) void chunk_call(const KJob& job, int64_t chunk, double* part,
                                                      int32_t* cf) {
-  chunk_body<D, FAM, GRID, COUPLED>(job, chunk, part, cf);
+  chunk_body<D, FAM, GRID, COUPLED, UF>(job, chunk, part, cf);
+}
+
+template <int D, int FAM, int GRID, bool COUPLED>
+__device__ __forceinline__ void chunk_case(const KJob& job, int64_t chunk, double* part,
+                                           int32_t* cf) {
+  if constexpr (GRID == SDEMC_GRID_UNIFORM && common_form<FAM>() != UFORM_ANY) {
+    if (takes_common_form<FAM>(job)) {
+      chunk_call<D, FAM, GRID, COUPLED, common_form<FAM>()>(job, chunk, part, cf);
+      return;
+    }
+  }
+  chunk_call<D, FAM, GRID, COUPLED, UFORM_ANY>(job, chunk, part, cf);
 }
 
 #define SDEMC_CASE(NOISE, D, FAM, GRID, C)                              \
   case ((NOISE * 4 + (D - 1)) * 2 + GRID) * 2 + C:                      \
-    chunk_call<D, FAM, GRID, (C != 0)>(job, chunk, part, cf);        \
+    chunk_case<D, FAM, GRID, (C != 0)>(job, chunk, part, cf);        \
     return true;
 
 #define SDEMC_CASES_DG(NOISE, D, FAM, GRID) \
@@ -125,7 +139,17 @@ __device__ __forceinline__ bool run_chunk(const KJob& job, int64_t chunk, double
                              ? (CLS == SDEMC_CLASS_INDEP2 ? 1 : 0)
                              : -1;
     if (MODE >= 0 && job.pois_mode != MODE) return false;
-    chunk_body<D, FAM, GRID, COUPLED, U, MODE>(job, chunk, part, cf);
+    // Both step forms stand in the dedicated uniform kernels: calling the
+    // general loop as a function cost the common one 20% (2-D: 2%) in saves
+    // around the call, and sending its jobs to the generic class 25-35% of
+    // their time.
+    if constexpr (GRID == SDEMC_GRID_UNIFORM) {
+      if (takes_common_form<FAM>(job)) {
+        chunk_body<D, FAM, GRID, COUPLED, common_form<FAM>(), U, MODE>(job, chunk, part, cf);
+        return true;
+      }
+    }
+    chunk_body<D, FAM, GRID, COUPLED, UFORM_ANY, U, MODE>(job, chunk, part, cf);
     return true;
   } else {
     switch (job.class_key) {

@@ -130,18 +130,61 @@ __device__ __forceinline__ void normals6(const U4& w, float* z) {
   const uint32_t wp[3] = {w.x, w.y, w.z};
 #pragma unroll
   for (int p = 0; p < 3; ++p) {
-    // 1 + a as float bits: 0x3F800000 | (w_p mod 2^9) << 14 | (w3 field) << 4
-    const uint32_t lo = (((w.w >> (10 * p)) & 0x3FFu) << 4) | 0x3F800000u;
-    const uint32_t bits = ((wp[p] << 14) & 0x007FC000u) | lo;
+    // 1 + a as float bits: 0x3F800000 | (w_p mod 2^9) << 14 | (w3 field) << 4,
+    // in two shifts, an and-or (1.0f is an inline constant) and a bit select
+    const uint32_t field = p == 0 ? w.w << 4 : w.w >> (10 * p - 4);
+    uint32_t lo, bits;
+    asm("v_and_or_b32 %0, %1, %2, 1.0" : "=v"(lo) : "v"(field), "s"(0x3FF0u));
+    asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(bits) : "s"(0x007FC000u), "v"(wp[p] << 14), "v"(lo));
     box_muller_ua(u01_open(wp[p]), __uint_as_float(bits), z[2 * p], z[2 * p + 1]);
   }
 }
 
-// Normals of block b of a path's Brownian stream.
-__device__ __forceinline__ void normal_block(uint32_t b, uint32_t plo, uint32_t phi, uint32_t k0,
-                                             uint32_t k1, float* z) {
-  normals6(philox4x32_10(b, STREAM_BM, plo, phi, k0, k1), z);
-}
+// A path's Brownian stream.  Its blocks differ in the counter word `block`, which
+// is the same for all lanes: the products of the first round are a scalar one
+// and one that depends on the path alone, and so is one product of the second,
+// so they are taken once per path or on the scalar unit, and a block costs 36
+// vector operations instead of 41 (philox4x32_10 bit for bit).
+struct BmStream {
+  uint32_t k0, k1;
+  uint32_t lo1;     // low word of 0xCD9E8D57 plo, xor the second round's key
+  uint32_t hiA, loA;  // the second round's product of the path's own word
+  uint32_t phi;
+  __device__ __forceinline__ void init(uint32_t key0, uint32_t key1, uint32_t plo, uint32_t hi) {
+    k0 = __builtin_amdgcn_readfirstlane(key0);
+    k1 = __builtin_amdgcn_readfirstlane(key1);
+    phi = hi;
+    const uint64_t p1 = (uint64_t)0xCD9E8D57u * plo;
+    const uint64_t pA = (uint64_t)0xD2511F53u * ((uint32_t)(p1 >> 32) ^ STREAM_BM ^ k0);
+    lo1 = (uint32_t)p1 ^ (k0 + 0x9E3779B9u);
+    hiA = (uint32_t)(pA >> 32);
+    loA = (uint32_t)pA;
+  }
+  __device__ __forceinline__ U4 block(uint32_t b) const {
+    uint32_t r0 = k0, r1 = k1;
+    asm volatile("" : "+s"(r0), "+s"(r1));  // the key schedule stays on the scalar unit
+    const uint64_t p0 = (uint64_t)0xD2511F53u * b;
+    const uint64_t p1 = (uint64_t)0xCD9E8D57u * (((uint32_t)(p0 >> 32) ^ r1) ^ phi);
+    r0 += 0x9E3779B9u;
+    r1 += 0xBB67AE85u;
+    uint32_t c0 = (uint32_t)(p1 >> 32) ^ lo1, c1 = (uint32_t)p1;
+    uint32_t c2 = hiA ^ ((uint32_t)p0 ^ r1), c3 = loA;
+#pragma unroll
+    for (int r = 2; r < 10; ++r) {
+      r0 += 0x9E3779B9u;
+      r1 += 0xBB67AE85u;
+      const uint64_t q0 = (uint64_t)0xD2511F53u * c0;
+      const uint64_t q1 = (uint64_t)0xCD9E8D57u * c2;
+      c0 = xor3_key((uint32_t)(q1 >> 32), c1, r0);
+      c1 = (uint32_t)q1;
+      c2 = xor3_key((uint32_t)(q0 >> 32), c3, r1);
+      c3 = (uint32_t)q0;
+    }
+    return U4{c0, c1, c2, c3};
+  }
+  // the six normals of block b
+  __device__ __forceinline__ void normals(uint32_t b, float* z) const { normals6(block(b), z); }
+};
 
 // Steps (or adapted-grid rows) whose K normals each are drawn together as
 // whole blocks: 4 when 4K normals fill whole blocks (K = 3), else 6.
@@ -200,21 +243,18 @@ __device__ __forceinline__ float ln_unit(uint32_t w) {
 // block i / 6 on the Brownian stream (normals6).  The last block is cached,
 // so sequential reads cost one Philox block per 6 normals.
 struct NormalStream {
-  uint32_t k0, k1, plo, phi;
+  BmStream bm;
   uint32_t blk;
   float z[NORMALS_PER_BLOCK];
   __device__ __forceinline__ void init(uint32_t key0, uint32_t key1, uint64_t path) {
-    k0 = key0;
-    k1 = key1;
-    plo = (uint32_t)path;
-    phi = (uint32_t)(path >> 32);
+    bm.init(key0, key1, (uint32_t)path, (uint32_t)(path >> 32));
     blk = 0xffffffffu;
   }
   __device__ __forceinline__ float get(uint32_t i) {
     const uint32_t b = i / (uint32_t)NORMALS_PER_BLOCK;
     if (b != blk) {
       blk = b;
-      normal_block(b, plo, phi, k0, k1, z);
+      bm.normals(b, z);
     }
     const uint32_t s = i - b * (uint32_t)NORMALS_PER_BLOCK;
     float v = z[0];
@@ -323,6 +363,27 @@ constexpr uint32_t KJOB_MAGIC = 0x5DE3C0DEu;
 // Dispatch key of a prepared job: ((noise * 4 + dim - 1) * 2 + grid) * 2 + coupled.
 inline int32_t class_key_of(int noise, int dim, int grid, bool coupled) {
   return ((noise * 4 + (dim - 1)) * 2 + grid) * 2 + (coupled ? 1 : 0);
+}
+
+// The folded uniform-grid step form of a model ('diag' and the jump solver's
+// 'indep' noise, no cross drift): every coefficient constant or every one
+// proportional to the state; UFORM_GENERIC otherwise.
+inline int32_t model_uform(const sdemc_model& m) {
+  if (m.noise != SDEMC_NOISE_DIAG && m.noise != SDEMC_NOISE_INDEP_COMMON) return UFORM_GENERIC;
+  bool cst = true, prop = true;
+  for (int i = 0; i < m.dim; ++i) {
+    if (m.ax[i] != 0.0) cst = prop = false;
+    if (m.a1[i] != 0.0 || m.b1[i] != 0.0 || m.c1[i] != 0.0) cst = false;
+    if (m.a0[i] != 0.0 || m.b0[i] != 0.0 || m.c0[i] != 0.0) prop = false;
+  }
+  return cst ? UFORM_CONST : (prop ? UFORM_PROP : UFORM_GENERIC);
+}
+
+// Constant jump coefficients.
+inline int32_t model_additive(const sdemc_model& m) {
+  for (int i = 0; i < m.dim; ++i)
+    if (m.j1[i] != 0.0) return 0;
+  return 1;
 }
 
 inline void make_kjob(const sdemc_job& j, KJob& k) {
@@ -438,35 +499,23 @@ inline void make_kjob(const sdemc_job& j, KJob& k) {
     const double mu = m.rate * j.T / (double)j.steps;
     if (mu >= POIS_MIN_MU) k.pois_mode = poisson_thresholds(mu, k.pois_T, k.pois_inv) ? 1 : 0;
   }
-  // Folded uniform-grid step constants ('diag' and the jump solver's 'indep'
-  // noise, no cross drift): every coefficient constant or every one
-  // proportional to the state.
-  k.uform = UFORM_GENERIC;
-  k.additive = 1;
-  for (int i = 0; i < m.dim; ++i)
-    if (m.j1[i] != 0.0) k.additive = 0;
+  // Folded uniform-grid step constants.
+  k.uform = model_uform(m);
+  k.additive = model_additive(m);
   for (int i = 0; i < SDEMC_MAX_DIM; ++i) {
     k.uA[i] = k.uC[i] = 0.0f;
     for (int q = 0; q < SDEMC_MAX_DIM; ++q) k.uW[i][q] = 0.0f;
   }
-  if (m.noise == SDEMC_NOISE_DIAG || m.noise == SDEMC_NOISE_INDEP_COMMON) {
-    bool cst = true, prop = true;
+  if (k.uform != UFORM_GENERIC) {
+    const bool cst = k.uform == UFORM_CONST;
+    const double h = (double)k.h, sq = sqrt(h);
     for (int i = 0; i < m.dim; ++i) {
-      if (m.ax[i] != 0.0) cst = prop = false;
-      if (m.a1[i] != 0.0 || m.b1[i] != 0.0 || m.c1[i] != 0.0) cst = false;
-      if (m.a0[i] != 0.0 || m.b0[i] != 0.0 || m.c0[i] != 0.0) prop = false;
-    }
-    if (cst || prop) {
-      k.uform = cst ? UFORM_CONST : UFORM_PROP;
-      const double h = (double)k.h, sq = sqrt(h);
-      for (int i = 0; i < m.dim; ++i) {
-        const double a = cst ? m.a0[i] : m.a1[i];
-        const double b = cst ? m.b0[i] : m.b1[i];
-        const double c = cst ? m.c0[i] : m.c1[i];
-        k.uA[i] = (float)(a * h);
-        k.uC[i] = m.noise == SDEMC_NOISE_INDEP_COMMON ? (float)(c * sq) : 0.0f;
-        for (int q = 0; q <= i; ++q) k.uW[i][q] = (float)(b * m.chol[i * SDEMC_MAX_DIM + q] * sq);
-      }
+      const double a = cst ? m.a0[i] : m.a1[i];
+      const double b = cst ? m.b0[i] : m.b1[i];
+      const double c = cst ? m.c0[i] : m.c1[i];
+      k.uA[i] = (float)(a * h);
+      k.uC[i] = m.noise == SDEMC_NOISE_INDEP_COMMON ? (float)(c * sq) : 0.0f;
+      for (int q = 0; q <= i; ++q) k.uW[i][q] = (float)(b * m.chol[i * SDEMC_MAX_DIM + q] * sq);
     }
   }
 }
@@ -1301,7 +1350,7 @@ struct CoarseAcc {
 // draws and the arithmetic are the same for every U).
 // POIS: the job's jump mode (per-step Poisson counts or the arrival clock),
 // a template parameter so each form keeps only its own state in registers;
-// path_uniform_rng below dispatches on the job.
+// as is UF, the job's step form (takes_common_form).
 // COUPLED: x is the fine path of an MLMC pair and xc (then non-null) its
 // coarse path, stepped every M = j.M fine steps by CoarseAcc.
 // UF: the step form the loop is compiled for (uniform_step).
@@ -1317,8 +1366,10 @@ __device__ void path_uniform_rng_form(const KJob& j, const PathCtx& c, bool lane
   const float sq = j.sqh;
   const uint32_t plo = (uint32_t)c.path, phi = (uint32_t)(c.path >> 32);
   constexpr bool pois = POIS;
+  BmStream bm;
+  bm.init(c.k0, c.k1, plo, phi);
   // the common forms' jump coefficients: the exponential Levy's are constant,
-  // the proportional ones are not (path_uniform_rng_mode asks for both)
+  // the proportional ones are not (takes_common_form asks for both)
   const bool additive = UF == UFORM_CONST ? true : (UF == UFORM_PROP ? false : j.additive != 0);
   JumpClock jc;
   int32_t kj = 0x7fffffff;
@@ -1425,7 +1476,11 @@ __device__ void path_uniform_rng_form(const KJob& j, const PathCtx& c, bool lane
     const uint32_t b0 = (uint32_t)n0 * (uint32_t)K / (uint32_t)NORMALS_PER_BLOCK;
 #pragma unroll
     for (int b = 0; b < G * K / NORMALS_PER_BLOCK; ++b)
-      normal_block(b0 + b, plo, phi, c.k0, c.k1, &z[NORMALS_PER_BLOCK * b]);
+      // (a coupled pair's general loop is short of registers: no products held)
+      if constexpr (COUPLED && UF == UFORM_ANY)
+        normals6(philox4x32_10(b0 + b, STREAM_BM, plo, phi, c.k0, c.k1), &z[NORMALS_PER_BLOCK * b]);
+      else
+        bm.normals(b0 + b, &z[NORMALS_PER_BLOCK * b]);
 #pragma unroll
     for (int s = 0; s < G; ++s) {
       const int32_t n = n0 + s;
@@ -1435,7 +1490,7 @@ __device__ void path_uniform_rng_form(const KJob& j, const PathCtx& c, bool lane
         if (COUPLED || (STORE && st.normals)) correlate<D, FAM>(f, &z[s * K], sq, dW, dB);
 #pragma unroll
         for (int i = 0; i < D; ++i) xo[i] = x[i];
-        uniform_step<D, FAM, UF>(j, x, &z[s * K], fine, uA);
+        uniform_step<D, FAM, UF>(j, x, &z[s * K], fine, UF == UFORM_PROP ? uA : j.uA);
         float jsum = 0.0f;
         // rare enough (and long) to be laid out of line: steps without a jump
         // run straight on
@@ -1573,15 +1628,18 @@ __device__ void path_uniform_rng_form(const KJob& j, const PathCtx& c, bool lane
       spill = __any(kj < wend);
     }
   };
+  // the general form of larger states keeps the end tests: without them the
+  // compiler holds more values across steps than the wavefronts pay for
+  using Full = std::bool_constant<!(UF == UFORM_ANY && D > (COUPLED ? 1 : 2))>;
   int32_t n0 = 0;
   for (; n0 + G * U <= N; n0 += G * U) {
     window(n0);
     if (spill) {
 #pragma unroll
-      for (int u = 0; u < U; ++u) group(n0 + G * u, std::true_type{}, std::true_type{});
+      for (int u = 0; u < U; ++u) group(n0 + G * u, std::true_type{}, Full{});
     } else {
 #pragma unroll
-      for (int u = 0; u < U; ++u) group(n0 + G * u, std::false_type{}, std::true_type{});
+      for (int u = 0; u < U; ++u) group(n0 + G * u, std::false_type{}, Full{});
     }
   }
   // the last steps of a grid that is no multiple of the stride
@@ -1591,34 +1649,23 @@ __device__ void path_uniform_rng_form(const KJob& j, const PathCtx& c, bool lane
   }
 }
 
-// The loop compiled for the family's common step form where the job has it
-// (storing kernels, bound by their writes, keep the general loop).  Told apart
-// in every step, the form, the end of the grid and the jump test were ten
-// scalar branches a step, which cost time even with eight wavefronts per SIMD:
-// 400 steps, 1-D GBM of 2^22 / 10^4 paths 954 -> 754 / 67 -> 33 us, 1-D Merton at
-// 2 jumps a path 1088 -> 831 / 85 -> 51 us, the 2-D Levy rainbow 3340 -> 2970 /
-// 199 -> 142 us.
-template <int D, int FAM, bool STORE, int U, bool POIS, bool COUPLED = false>
-__device__ __forceinline__ void path_uniform_rng_mode(const KJob& j, const PathCtx& c,
-                                                      bool lane_valid, float (&x)[D],
-                                                      const StoreCtx& st, float* xc = nullptr) {
-  constexpr int UF = STORE ? UFORM_ANY : common_form<FAM>();
-  if constexpr (UF != UFORM_ANY) {
-    if (j.uform == UF && (j.m.rate == 0.0 || (j.additive != 0) == (UF == UFORM_CONST))) {
-      path_uniform_rng_form<D, FAM, STORE, U, POIS, COUPLED, UF>(j, c, lane_valid, x, st, xc);
-      return;
-    }
-  }
-  path_uniform_rng_form<D, FAM, STORE, U, POIS, COUPLED>(j, c, lane_valid, x, st, xc);
+__host__ __device__ constexpr bool is_common_form(int form, int32_t uform, int32_t additive,
+                                                  double rate) {
+  return form != UFORM_ANY && uform == form &&
+         (rate == 0.0 || (additive != 0) == (form == UFORM_CONST));
 }
 
-template <int D, int FAM, bool STORE, int U = 1>
-__device__ __forceinline__ void path_uniform_rng(const KJob& j, const PathCtx& c, bool lane_valid,
-                                                 float (&x)[D], const StoreCtx& st) {
-  if (j.pois_mode != 0)
-    path_uniform_rng_mode<D, FAM, STORE, U, true>(j, c, lane_valid, x, st);
-  else
-    path_uniform_rng_mode<D, FAM, STORE, U, false>(j, c, lane_valid, x, st);
+// Whether the job has its family's common step form: kernels hold the loop of
+// one form each (a kernel body with both keeps the registers of the larger).
+// Told apart in every step, the form, the end of the grid and the jump test
+// were ten scalar branches a step, which cost time even with eight wavefronts
+// per SIMD: 400 steps, 1-D GBM of 2^22 / 10^4 paths 954 -> 754 / 67 -> 33 us, 1-D
+// Merton at 2 jumps a path 1088 -> 831 / 85 -> 51 us, the 2-D Levy rainbow 3340 ->
+// 2970 / 199 -> 142 us.  Storing kernels, bound by their writes, run the
+// general loop.
+template <int FAM>
+__host__ __device__ __forceinline__ bool takes_common_form(const KJob& j) {
+  return is_common_form(common_form<FAM>(), j.uform, j.additive, j.m.rate);
 }
 
 // Coupled fine/coarse pair on the uniform grid (an MLMC level), Philox
@@ -1626,14 +1673,11 @@ __device__ __forceinline__ void path_uniform_rng(const KJob& j, const PathCtx& c
 // it shares the 4-step normal blocks, the jump queue and the per-wavefront
 // jump lists; the draws, their order and the arithmetic are those of
 // path_uniform_coupled.
-template <int D, int FAM, int U = 1>
+template <int D, int FAM, bool POIS, int UF>
 __device__ __forceinline__ void path_uniform_rng_coupled(const KJob& j, const PathCtx& c,
                                                          float (&xf)[D], float (&xc)[D]) {
   const StoreCtx st{};
-  if (j.pois_mode != 0)
-    path_uniform_rng_mode<D, FAM, false, U, true, true>(j, c, true, xf, st, xc);
-  else
-    path_uniform_rng_mode<D, FAM, false, U, false, true>(j, c, true, xf, st, xc);
+  path_uniform_rng_form<D, FAM, false, 1, POIS, true, UF>(j, c, true, xf, st, xc);
 }
 
 // Row layout of fixed increments per step: D ('diag'), D + 1 ('indep'
@@ -1936,6 +1980,7 @@ struct AdaptQueueSrc {
   static constexpr bool SORTED = true;  // jump times never decrease
   JumpClock jc;                         // the last jump drawn
   uint32_t plo, phi, k0, k1, lane;
+  BmStream bm;
   uint32_t head;
   ClockLds* cq;
   __device__ __forceinline__ void put(const KModel& f) {
@@ -1969,6 +2014,7 @@ struct AdaptQueueSrc {
     k1 = c.k1;
     plo = (uint32_t)c.path;
     phi = (uint32_t)(c.path >> 32);
+    bm.init(k0, k1, plo, phi);
     lane = __lane_id();
     cq = reinterpret_cast<ClockLds*>(&pois_lds());
     head = 0;
@@ -1990,7 +2036,7 @@ struct AdaptQueueSrc {
     const uint32_t b0 = row0 * (uint32_t)K / (uint32_t)NORMALS_PER_BLOCK;
 #pragma unroll
     for (int b = 0; b < G * K / NORMALS_PER_BLOCK; ++b)
-      normal_block(b0 + b, plo, phi, k0, k1, &zq[NORMALS_PER_BLOCK * b]);
+      bm.normals(b0 + b, &zq[NORMALS_PER_BLOCK * b]);
   }
   __device__ __forceinline__ float next_time(bool = true) const {
     return __int_as_float(cq->k[head % CLOCK_JQ][lane]);

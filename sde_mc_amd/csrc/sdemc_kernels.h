@@ -9,9 +9,14 @@ namespace sdemc {
 
 // Plain RNG-mode kernel: one wavefront per 64-path chunk.  Paths, payoff and
 // the chunk's fp64 partial sums in one pass; per-path outputs are optional.
-// POIS: the uniform single-level path's jump mode (the job's pois_mode), so
-// each kernel holds the registers of one mode only.
-template <int D, int FAM, int GRID, bool COUPLED, bool STORE, bool POIS = false>
+// POIS: the uniform path's jump mode (the job's pois_mode), UF: its step form
+// (the family's common one or the general), so each kernel holds the
+// registers of one loop only: with both forms in one kernel, coupled pairs of
+// two or more components lost more to their registers than the common form
+// gained (2^20 pairs x 400 fine steps, 2-D Merton 684 us before there were two
+// forms, 772 with both, 612 as separate kernels; 2-D Levy 1190 / 1286 / 1057).
+template <int D, int FAM, int GRID, bool COUPLED, bool STORE, bool POIS = false,
+          int UF = UFORM_ANY>
 __global__ __launch_bounds__(512) void k_rng(const KJob job, double* __restrict__ partials,
                                              int32_t* __restrict__ cflags,
                                              const sdemc_path_out out, int64_t nchunks) {
@@ -42,7 +47,7 @@ __global__ __launch_bounds__(512) void k_rng(const KJob job, double* __restrict_
   if (!COUPLED) {
     float x[D];
     if (GRID == SDEMC_GRID_UNIFORM) {
-      path_uniform_rng_mode<D, FAM, STORE, STORE ? 1 : 2, POIS>(job, c, valid, x, st);
+      path_uniform_rng_form<D, FAM, STORE, STORE ? 1 : 2, POIS, false, UF>(job, c, valid, x, st);
     } else {
       AdaptQueueSrc<D, FAM> src;
       src.init(job.m, c);
@@ -58,7 +63,7 @@ __global__ __launch_bounds__(512) void k_rng(const KJob job, double* __restrict_
   } else {
     float xf[D], xc[D];
     if (GRID == SDEMC_GRID_UNIFORM) {
-      path_uniform_rng_coupled<D, FAM>(job, c, xf, xc);
+      path_uniform_rng_coupled<D, FAM, POIS, UF>(job, c, xf, xc);
     } else {
       AdaptQueueSrc<D, FAM> src;
       src.init(job.m, c);
@@ -313,33 +318,34 @@ int launch_rng_d(const sdemc_job& sj, const LaunchArgs& a) {
   const dim3 g((unsigned)blocks), b((unsigned)threads);
   // the per-wavefront jump lists of the uniform grid's per-step Poisson mode
   const size_t lds = (size_t)a.wpb * sizeof(PoisLds);
-#define SDEMC_L(G, C, S)                                                                     \
-  hipLaunchKernelGGL((k_rng<D, FAM, G, C, S>), g, b, lds, a.stream, job, a.partials, a.cflags,    \
-                     a.out, nchunks)
-#define SDEMC_LU(S)                                                                           \
-  if (job.pois_mode)                                                                          \
-    hipLaunchKernelGGL((k_rng<D, FAM, SDEMC_GRID_UNIFORM, false, S, true>), g, b, lds, a.stream, \
-                       job, a.partials, a.cflags, a.out, nchunks);                            \
-  else                                                                                        \
-    SDEMC_L(SDEMC_GRID_UNIFORM, false, S)
+#define SDEMC_L(G, C, S, ...)                                                                 \
+  hipLaunchKernelGGL((k_rng<D, FAM, G, C, S, ##__VA_ARGS__>), g, b, lds, a.stream, job,       \
+                     a.partials, a.cflags, a.out, nchunks)
+#define SDEMC_LU(C, S, UF)                                                                    \
+  if (job.pois_mode) SDEMC_L(SDEMC_GRID_UNIFORM, C, S, true, UF);                             \
+  else SDEMC_L(SDEMC_GRID_UNIFORM, C, S, false, UF)
   if constexpr (FAM == FAM_DOUBLE || FAM == FAM_HESTON || FAM == FAM_GENERAL) {
     if (adapted) return SDEMC_ERR_UNSUPPORTED;
-    if (coupled) SDEMC_L(SDEMC_GRID_UNIFORM, true, false);
-    else if (a.store) { SDEMC_LU(true); }
-    else { SDEMC_LU(false); }
+    if (coupled) { SDEMC_LU(true, false, UFORM_ANY); }
+    else if (a.store) { SDEMC_LU(false, true, UFORM_ANY); }
+    else { SDEMC_LU(false, false, UFORM_ANY); }
   } else {
+    // storing kernels, bound by their writes, keep the general loop
+    const bool common = takes_common_form<FAM>(job);
     if (!coupled) {
       if (!adapted) {
-        if (a.store) { SDEMC_LU(true); }
-        else { SDEMC_LU(false); }
+        if (a.store) { SDEMC_LU(false, true, UFORM_ANY); }
+        else if (common) { SDEMC_LU(false, false, common_form<FAM>()); }
+        else { SDEMC_LU(false, false, UFORM_ANY); }
       } else {
         if (a.store) SDEMC_L(SDEMC_GRID_ADAPTED, false, true);
         else SDEMC_L(SDEMC_GRID_ADAPTED, false, false);
       }
     } else {
       if (a.store) return SDEMC_ERR_UNSUPPORTED;
-      if (!adapted) SDEMC_L(SDEMC_GRID_UNIFORM, true, false);
-      else SDEMC_L(SDEMC_GRID_ADAPTED, true, false);
+      if (adapted) SDEMC_L(SDEMC_GRID_ADAPTED, true, false);
+      else if (common) { SDEMC_LU(true, false, common_form<FAM>()); }
+      else { SDEMC_LU(true, false, UFORM_ANY); }
     }
   }
 #undef SDEMC_L
