@@ -196,19 +196,29 @@ __device__ __forceinline__ void raise_fault(int32_t* fault, int lane) {
   if (lane == 0) *fault = 1;
 }
 
-// Persistent tile kernel of one class group.  hdr = {first segment,
-// segments, tiles}; tile indices come from this group's counter.  U is the
-// step unroll of the uniform single-level path (classes 0, 4 and 8).
 // Wavefronts per SIMD: the dedicated class kernels are held to 64 VGPRs so
 // that 8 fit (the served mix's per-step count kernel went from 66 VGPRs, 7
 // wavefronts, to 64 with 20 B of spills per lane, and the round from 41.4 to
-// 39.7 ms; the coupled and adapted classes move by -7% .. +2%); the generic
-// class, whose cases' register needs go up to ~250 VGPRs for the 4-D
+// 39.7 ms; the adapted classes move by -4% .. +2%); the uniform coupled
+// classes, whose two halves and two step forms need more, to 72 (1-D) and 80
+// (2-D): at 64 they spilled 112 and 172 B a lane (4e5 pairs x 200 fine steps,
+// 2-D Levy 532 -> 511 us, its general form 607 -> 576; 1-D Merton 332 -> 323);
+// the generic class, whose cases' register needs go up to ~250 VGPRs for the 4-D
 // two-driver family, to 128 (4 wavefronts; a few of its cases spill a
 // little) instead of running at 2 per SIMD.
+constexpr int batch_waves(int cls) {
+  if (cls == SDEMC_CLASS_GENERIC) return 4;
+  if (cls == SDEMC_CLASS_DIAG1 + 1) return 7;
+  if (cls == SDEMC_CLASS_INDEP2 + 1) return 6;
+  return 8;
+}
+
+// Persistent tile kernel of one class group.  hdr = {first segment,
+// segments, tiles}; tile indices come from this group's counter.  U is the
+// step unroll of the uniform single-level path (classes 0, 4 and 8).
 template <int CLS, int U>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
-    CLS == SDEMC_CLASS_GENERIC ? 4 : 8))) void k_batch(const KJob* __restrict__ jobs,
+    batch_waves(CLS)))) void k_batch(const KJob* __restrict__ jobs,
                                                const sdemc_segment* __restrict__ segs,
                                                const int32_t* __restrict__ hdr,
                                                double* __restrict__ partials,
