@@ -34,13 +34,16 @@ constexpr int CV_BLOCK_WORDS = 512;  // one operand fragment: 64 lanes x 8 bf16
 constexpr int CV_MAX_THREADS = 512;
 
 // Wavefronts per workgroup.  The workgroup's wavefronts share one LDS copy of
-// the weights (22 KB for a network of three hidden layers), so eight of them
-// leave room for the four wavefronts per SIMD that the registers allow where
-// workgroups of four with both networks fit three; a launch of fewer chunks
-// takes smaller workgroups, so that it reaches all 256 CUs.  2^18 Merton paths x
-// 300 adapted steps with an f and a g: 2782 -> 2613 us.
+// the weights (22 KB for a network of three hidden layers): workgroups of eight
+// leave room for the sixteen wavefronts a CU that the registers allow where
+// workgroups of four with both networks fit three.  That pays while the
+// launch fits the chip at once (2^18 Merton paths x 300 adapted steps with an f
+// and a g: 2782 -> 2613 us); over several rounds the matrix cores are busy
+// either way and the smaller workgroups hand over sooner (2^20 x 1000: 28.6 ms
+// with four, 29.4 with eight).  A launch of few chunks takes smaller ones,
+// so that it reaches all 256 CUs.
 inline int cv_waves_per_block(int64_t nchunks) {
-  int w = 8;
+  int w = nchunks <= 256 * 16 ? 8 : 4;
   while (w > 1 && nchunks < 256 * (int64_t)w) w >>= 1;
   return w;
 }
