@@ -710,7 +710,9 @@ __device__ __forceinline__ void euler(const KModel& f, float (&x)[D], float dt,
 
 // The Heston step of a fixed step size, carrying sqrt(v): euler<2, FAM_HESTON>
 // bit for bit.  The new v is y^2 rounded, and the root of a rounded square is the
-// number itself, so the next step's sqrt(v) is y; the divisor 2 A is the same
+// number's magnitude (while the square neither over- nor underflows), so the next
+// step's sqrt(v) is |y|: y itself but where the constant term is lost beside B^2,
+// B < 0 and the hardware root leaves y one unit below zero; the divisor 2 A is the same
 // every step, and with its correctly rounded reciprocal r one residual step
 // rounds n / (2 A) correctly (Markstein, IBM J. Res. Dev. 34, 1990): one root and
 // three operations for the quotient instead of two roots and a full division.
@@ -736,7 +738,7 @@ struct HestonStep {
     const float B = f.hv_xi * dW[1];
     const float n = B + __builtin_amdgcn_sqrtf(__fmaf_rn(B, B, A4 * C));
     const float q = n * r;
-    sv = __fmaf_rn(__fmaf_rn(-den, q, n), r, q);
+    sv = __builtin_fabsf(__fmaf_rn(__fmaf_rn(-den, q, n), r, q));
     x[1] = sv * sv;
   }
 };
