@@ -250,7 +250,9 @@ class DeviceNetwork:
         plan = layer_plan(model)
         _check_shape(plan, n_in, n_out)
         self.hidden = len(plan) - 1
-        entries, held = _device_layers(plan, device)
+        # parameters on the host, wherever the words go: the host packs
+        on_device = torch.device(device).type == 'cuda'
+        entries, held = _device_layers(plan, device) if on_device else (None, None)
         if entries is None:
             arr, self.hidden = pack_network(model, n_in, n_out)
             self.words = torch.from_numpy(arr.view(np.int16).copy()).to(device)
