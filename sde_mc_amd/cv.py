@@ -189,49 +189,54 @@ class ZeroNetwork:
 
 
 def _check_shape(plan, n_in, n_out):
-    """The limits of the packed form (padded_matrices)."""
+    """The limits of the packed form (padded_matrices), by the weights' own shapes."""
     if len(plan) - 1 > MAX_HIDDEN:
         raise NotImplementedError('at most %d hidden layers' % MAX_HIDDEN)
-    if plan[0][0].in_features != n_in or plan[-1][0].out_features != n_out:
+    if plan[0][0].weight.shape[1] != n_in or plan[-1][0].weight.shape[0] != n_out:
         raise NotImplementedError('network must map R^%d to R^%d' % (n_in, n_out))
     if n_in + 1 > 8 or n_out > MAX_OUT:
         raise NotImplementedError('at most 7 inputs and %d outputs' % MAX_OUT)
-    if any(lin.out_features > HIDDEN_PAD - 1 for lin, _, _ in plan[:-1]):
+    if any(lin.weight.shape[0] > HIDDEN_PAD - 1 for lin, _, _ in plan[:-1]):
         raise NotImplementedError('hidden layers of at most %d units' % (HIDDEN_PAD - 1))
 
 
 def _device_layers(plan, device):
     """The plan as sdemc_cv_layer entries when every parameter is an fp32
-    tensor on `device` that the packing kernel can read, else None (the host
-    packs then).  The second value holds the tensors the entries point into."""
+    tensor on `device` of the size its place in the network gives it, which is
+    all the packing kernel reads, else None (the host packs then, or refuses).
+    The second value holds the tensors the entries point into."""
     held = []
 
-    def ptr(t):
+    def ptr(t, *shape):
         if t is None:
             return None
         t = t.detach()
-        if t.dtype != torch.float32 or t.device != device or t.layout != torch.strided:
+        if t.dtype != torch.float32 or t.device != device or t.layout != torch.strided \
+                or tuple(t.shape) != shape:
             raise TypeError
         held.append(t.contiguous())
         return held[-1].data_ptr()
 
-    def bn(m):
+    def bn(m, width):
         e = CvBn()
         if m is not None:
             if m.running_var is None or m.running_mean is None:
                 raise TypeError
-            e.weight_dev, e.bias_dev = ptr(m.weight), ptr(m.bias)
-            e.mean_dev, e.var_dev, e.eps = ptr(m.running_mean), ptr(m.running_var), float(m.eps)
+            e.weight_dev, e.bias_dev = ptr(m.weight, width), ptr(m.bias, width)
+            e.mean_dev, e.var_dev = ptr(m.running_mean, width), ptr(m.running_var, width)
+            e.eps = float(m.eps)
         return e
 
     entries = (CvLayer * len(plan))()
+    width = plan[0][0].weight.shape[1]
     try:
         for e, (lin, pre, post) in zip(entries, plan):
             if len(post) > 1:
                 return None, None
-            e.weight_dev, e.bias_dev = ptr(lin.weight), ptr(lin.bias)
-            e.n_in, e.n_out = lin.in_features, lin.out_features
-            e.pre, e.post = bn(pre), bn(post[0] if post else None)
+            e.n_in, e.n_out = width, lin.weight.shape[0]
+            e.weight_dev, e.bias_dev = ptr(lin.weight, e.n_out, width), ptr(lin.bias, e.n_out)
+            e.pre, e.post = bn(pre, width), bn(post[0] if post else None, e.n_out)
+            width = e.n_out
     except TypeError:
         return None, None
     return entries, held
