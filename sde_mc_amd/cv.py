@@ -249,6 +249,7 @@ class DeviceNetwork:
 
     def __init__(self, model, n_in, n_out, device):
         self.n_out = n_out
+        self._stream = None   # of the packing launch, and its end
         if model is None or is_zero_network(model):
             self.hidden, self.words = 0, None
             return
@@ -266,8 +267,18 @@ class DeviceNetwork:
         L.check(L.lib().sdemc_cv_pack(entries, len(plan), n_in, n_out, E.ptr(self.words),
                                       E.stream_ptr()), 'sdemc_cv_pack')
         del held   # freed in stream order after the launch
+        self._stream = torch.cuda.current_stream()
+        self._packed = self._stream.record_event()
 
     def c(self):
+        """The C descriptor, for a launch on the current stream: ordered after
+        the packing launch when that ran on another (a captured stream cannot
+        wait on work outside its graph; the capture begins synchronised)."""
+        if self._stream is not None and not torch.cuda.is_current_stream_capturing():
+            stream = torch.cuda.current_stream()
+            if stream != self._stream:
+                stream.wait_event(self._packed)
+                self.words.record_stream(stream)
         m = CvMlp()
         m.weights_dev = self.words.data_ptr() if self.words is not None else None
         m.hidden_layers = self.hidden
