@@ -41,12 +41,12 @@ class _Linear(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dy):
         x, weight = ctx.saved_tensors
-        dx = dw = db = None
-        if ctx.needs_input_grad[0]:
-            dx = dy @ weight
-        if ctx.needs_input_grad[1] or ctx.needs_input_grad[2]:
-            dw, db = E.linear_grads(x, dy.contiguous())
-        return dx, dw, db if ctx.needs_input_grad[2] else None
+        for_x, for_w, for_b = ctx.needs_input_grad
+        dx = dy @ weight if for_x else None
+        if torch.is_grad_enabled():   # gradients of these gradients are wanted: torch's own graph
+            return dx, dy.t() @ x if for_w else None, dy.sum(0) if for_b else None
+        dw, db = E.linear_grads(x, dy.contiguous()) if for_w or for_b else (None, None)
+        return dx, dw if for_w else None, db if for_b else None
 
 
 def _plain_linear(m):
