@@ -60,13 +60,13 @@ def _training_forward(model):
     the device.  Only what a training step does passes through it (first-order
     gradients of a plain module): a subclass, hooks, autocast or a
     non-standard layer keep the module's own call."""
-    mods = [model, model.net] + list(model.net) if type(model) is Mlp else []
+    plain = type(model) is Mlp and type(model.net) is torch.nn.Sequential
+    mods = [model, model.net] + list(model.net) if plain else []
     hooked = any(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks
                  or m._backward_pre_hooks or 'forward' in m.__dict__ for m in mods) or any(
         getattr(torch.nn.modules.module, '_global_%s_hooks' % k)
         for k in ('forward', 'forward_pre', 'backward', 'backward_pre'))
-    if not mods or hooked or not any(_plain_linear(m) for m in mods) or \
-            type(model.net) is not torch.nn.Sequential:
+    if hooked or not any(_plain_linear(m) for m in mods):
         return model
 
     def forward(x):
