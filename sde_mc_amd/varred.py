@@ -50,8 +50,9 @@ class _Linear(torch.autograd.Function):
 
 
 def _plain_linear(m):
-    return (type(m) is torch.nn.Linear and m.weight.is_cuda and m.weight.dtype == torch.float32
-            and m.in_features <= 63 and m.out_features <= 64)
+    w = m.weight if type(m) is torch.nn.Linear else None
+    return (type(w) is torch.nn.Parameter and w.is_cuda and w.dtype == torch.float32
+            and w.shape[0] <= 64 and w.shape[1] <= 63)
 
 
 def _training_forward(model):
