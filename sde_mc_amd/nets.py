@@ -9,7 +9,7 @@ evaluated by torch on stored paths.
 import torch
 import torch.nn as nn
 import torch.optim as optim
-from torch.utils.data import DataLoader, Dataset
+from torch.utils.data import DataLoader, Dataset, default_collate
 
 from . import engine as E
 
@@ -168,9 +168,16 @@ class AdaptedPathData(Dataset):
 class PathLoader(DataLoader):
     """DataLoader over a path dataset whose batches are gathered array by array
     (dataset.gather) instead of being stacked from single trajectories: the
-    same batches in the same order (no workers)."""
+    same batches in the same order.  One without batches, or with workers,
+    pinned memory or a collate_fn of its own is a plain DataLoader."""
 
     def __iter__(self):
+        if (self.batch_sampler is None or self.num_workers or self.pin_memory
+                or self.collate_fn is not default_collate):
+            return super().__iter__()
+        return self._gathered()
+
+    def _gathered(self):
         # a DataLoader takes its workers' base seed from the generator before
         # the sampler takes its own: kept, so a seed gives the same shuffle
         torch.empty((), dtype=torch.int64).random_(generator=self.generator)
