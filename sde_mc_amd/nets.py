@@ -175,14 +175,11 @@ class PathLoader(DataLoader):
         if (self.batch_sampler is None or self.num_workers or self.pin_memory
                 or self.collate_fn is not default_collate):
             return super().__iter__()
-        return self._gathered()
-
-    def _gathered(self):
-        # a DataLoader takes its workers' base seed from the generator before
-        # the sampler takes its own: kept, so a seed gives the same shuffle
+        # a DataLoader takes its workers' base seed from the generator when the
+        # iteration is asked for, and the sampler its own at the first batch:
+        # kept, so a seed gives the same shuffle
         torch.empty((), dtype=torch.int64).random_(generator=self.generator)
-        for index in self.batch_sampler:
-            yield self.dataset.gather(index)
+        return (self.dataset.gather(index) for index in self.batch_sampler)
 
 
 def get_mlps(problem, num_layers, hidden_size, device):

@@ -40,3 +40,16 @@ def test_workers_are_used():
     it = iter(dl)
     assert type(it).__module__.startswith('torch.utils.data')
     del it
+
+
+@pytest.mark.parametrize('generator', [False, True])
+def test_seed_between_the_iteration_and_its_first_batch(generator):
+    ds = _data()
+    order = []
+    for cls in (DataLoader, PathLoader):
+        g = torch.Generator().manual_seed(8) if generator else None
+        torch.manual_seed(1)
+        it = iter(cls(ds, batch_size=4, shuffle=True, generator=g))
+        torch.manual_seed(2)
+        order.append([payoffs for _, payoffs in it] + [torch.rand(2)])
+    assert all(torch.equal(a, b) for a, b in zip(*order))
