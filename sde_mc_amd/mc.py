@@ -22,6 +22,7 @@ from . import engine as E
 from .helpers import ceil_mult, mc_estimates, remove_steps, sample_cov
 from .nets import AdaptedPathData, NormalPathData, PathLoader
 from .options import ConstantShortRate
+from .solvers import SdeSolver
 from .varred import (EarlyStopping, apply_adapted_control_variates,
                      apply_diffusion_control_variate, train_adapted_control_variates,
                      train_diffusion_control_variate)
@@ -65,7 +66,8 @@ def mc_simple(num_trials, sde_solver, payoff, discounter=None, bs=None, return_n
     they fit in ``max_path_bytes``.  With ``bs`` only the fp64 sums come back:
     a payoff the kernels evaluate needs no storage per path, so its batches run
     as one launch each of at least FUSED_LAUNCH paths; any other payoff is
-    applied in torch to ``bs`` terminal states at a time.  The payoff is always taken
+    applied in torch to ``bs`` terminal states at a time, and a solver with a
+    simulate_stats of its own is asked for ``bs`` paths at a time.  The payoff is always taken
     at the terminal time: the reference's payoff_time='terminal' reads column
     num_steps of a jump-adapted path, which is an earlier state whenever a
     path jumped (mc.py:84-85); 'adapted' (mc.py:90-91) is what is computed.
@@ -92,7 +94,9 @@ def mc_simple(num_trials, sde_solver, payoff, discounter=None, bs=None, return_n
         od = sde_solver._out_device()
         return MCStatistics(mn, se, tt, num_trials, out, payoffs.to(od), normals)
     bs = int(bs)
-    if payoff.kernel_payoff(L.Payoff()):
+    # the solver's own fused run stores nothing per path; another's may
+    own = getattr(sde_solver.simulate_stats, '__func__', None) is SdeSolver.simulate_stats
+    if own and payoff.kernel_payoff(L.Payoff()):
         bs = max(bs, FUSED_LAUNCH)
     remaining = num_trials
     s = q = 0.0
