@@ -160,8 +160,9 @@ def gather_paths(arrays, index):
         and a.shape[0] == n and a.dim() <= 4 and not a.requires_grad for a in arrays)
     shapes = [_rows_and_dim(a) for a in arrays] if one else [None]
     if any(s is None for s in shapes):
-        idx = torch.as_tensor(index, dtype=torch.int64, device=dev)
-        return [a[idx].contiguous() for a in arrays]
+        idx = torch.as_tensor(index, dtype=torch.int64)
+        idx = {d: idx.to(d) for d in {a.device for a in arrays}}
+        return [a[idx[a.device]].contiguous() for a in arrays]
     if len(index) and not (0 <= min(index) and max(index) < n):
         raise IndexError('path index out of range')
     idx = torch.tensor(index, dtype=torch.int64).to(dev)
