@@ -397,8 +397,9 @@ int sdemc_linear_grads(const float* x_dev, const float* dy_dev, int64_t rows, in
  * cut into tiles of `per_tile` chunks; segment s owns tiles
  * [tile_begin, tile_begin + ceil(count / per_tile)), the segments' tile
  * ranges are consecutive from 0, and the list order is the order in which
- * tiles are handed out.  Persistent wavefronts take tile indices from a
- * device counter until all tiles are taken, so jobs of any size and any mix
+ * tiles are handed out.  Persistent wavefronts take the tile of their own
+ * number and then tile indices from a device counter until all tiles are
+ * taken, so jobs of any size and any mix
  * of models, grids and MLMC levels share one launch.  Partials of slot j
  * live at partials[chunk_base_j + c].  A launch whose segments name an
  * unprepared slot, chunks outside a slot or the partial pool, or tile ranges
@@ -447,9 +448,10 @@ int sdemc_prepare_jobs(const sdemc_job* jobs, int32_t n, const int64_t* chunk_ba
 
 /* A launch runs n_groups persistent kernels in stream order, one per class
  * group; group g's segments are segs[hdr[g][0] .. hdr[g][0] + hdr[g][1])
- * with hdr[g][2] tiles, taken from counter[g].  A segment whose job is not
- * of the group's class is refused in the kernel (NaN partials, chunk
- * flag 4) instead of being computed by the wrong code. */
+ * with hdr[g][2] tiles, the first of them taken by wavefront number and the
+ * others from counter[g].  A segment whose job is not of the group's class is
+ * refused in the kernel (NaN partials, chunk flag 4) instead of being computed
+ * by the wrong code. */
 typedef struct sdemc_batch_dev {
   const void* jobs_dev;          /* [max_jobs] prepared slots                   */
   const sdemc_segment* segs_dev; /* [max_segments], each group's contiguous     */

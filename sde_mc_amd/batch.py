@@ -8,11 +8,11 @@ first tile) -- grouped by kernel class, and the mask of slots to finalise.
 Each class group runs in its own persistent kernel, specialised to one
 (model family, time grid, single level or coupled pair) exactly like the
 plain launch's kernel for it, or the generic kernel for anything else; its
-wavefronts take tile indices from the group's device counter until the
-group's tiles are exhausted.  The launches of a round (counter reset, the
-group kernels, finalisation) are captured once per (round buffer, class
-groups) in a HIP graph and replayed; the host only uploads the small
-segment list and, for new jobs, their slots.
+wavefronts each run the tile of their own number, then take tile indices from
+the group's device counter until the group's tiles are exhausted.  The
+launches of a round (counter reset, the group kernels, finalisation) are
+captured once per (round buffer, class groups) in a HIP graph and replayed;
+the host only uploads the small segment list and, for new jobs, their slots.
 
 A job's result is independent of what it is packed with or how it is cut:
 the Philox streams are keyed by (seed, path) and the reduction order is
@@ -133,7 +133,7 @@ class RoundPlan:
 
 
 # Least work of one tile, in job_cost units (about 300 steps of a 1-D chunk):
-# a wavefront takes a tile index from its group's counter with one atomic, so
+# a wavefront takes its later tile indices from its group's counter, one atomic each, so
 # short jobs (e.g. MLMC level 0, 4 steps) get several chunks per tile.
 MIN_TILE_COST = 2.0e4
 MAX_TILE_COST = 5.0e4

@@ -1,7 +1,8 @@
 // k_batch.hip -- the batched persistent launch: one kernel runs a segment
 // list spanning any number of jobs (different models, grids, path counts,
-// step counts and MLMC levels).  Each wavefront repeatedly takes the next
-// tile index from a device counter and finds its segment by binary search,
+// step counts and MLMC levels).  Each wavefront runs the tile of its own
+// number, then takes further tile indices from a device counter, and finds a
+// tile's segment by binary search,
 // so long and short tiles balance across the 256 CUs without host
 // involvement; the host orders segments costliest-first.
 #include <string.h>

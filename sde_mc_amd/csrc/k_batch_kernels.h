@@ -214,8 +214,15 @@ constexpr int batch_waves(int cls) {
 }
 
 // Persistent tile kernel of one class group.  hdr = {first segment,
-// segments, tiles}; tile indices come from this group's counter.  U is the
-// step unroll of the uniform single-level path (classes 0, 4 and 8).
+// segments, tiles}.  A wavefront's first tile is its own number (the blocks'
+// first wavefronts before their second, so few tiles lie on many CUs), the
+// later ones come from this group's counter: one device address takes 12 ns an
+// atomic, and with every wavefront's first tile taken there too a launch of 7168
+// wavefronts spent 86 us on it before the longest tile counted, with the code
+// and constants of the larger loops waiting for the same cache behind the queue
+// (4e5 paths x 96 steps, 2-D Levy clock / 1-D Merton 196 / 161 -> 123 / 97 us; 2e4
+// paths 125 / 92 -> 47 / 29).  U is the step unroll of the uniform single-level
+// path (classes 0, 4 and 8).
 template <int CLS, int U>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
     batch_waves(CLS)))) void k_batch(const KJob* __restrict__ jobs,
@@ -242,11 +249,14 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
   }
   int32_t seg = s0;
   const int32_t last = s0 + nseg - 1;
-  for (;;) {
-    int32_t t = 0;
-    if (lane == 0) t = atomicAdd(counter, 1);
-    t = __shfl(t, 0);
-    t = __builtin_amdgcn_readfirstlane(t);
+  const int32_t waves = (int32_t)(gridDim.x * (blockDim.x / WAVE));
+  int32_t t = __builtin_amdgcn_readfirstlane(
+      (int32_t)((threadIdx.x / WAVE) * gridDim.x + blockIdx.x));
+  for (bool first = true;; first = false) {
+    if (!first) {
+      if (lane == 0) t = atomicAdd(counter, 1);
+      t = waves + __builtin_amdgcn_readfirstlane(t);
+    }
     if (t >= ntiles) break;
     // segment owning tile t: the last one whose tile_begin <= t; a wave's
     // tile indices only grow, so search [seg, last]
