@@ -196,21 +196,21 @@ __device__ __forceinline__ void raise_fault(int32_t* fault, int lane) {
   if (lane == 0) *fault = 1;
 }
 
-// Wavefronts per SIMD: the dedicated class kernels are held to 64 VGPRs so
-// that 8 fit (the served mix's per-step count kernel went from 66 VGPRs, 7
-// wavefronts, to 64 with 20 B of spills per lane, and the round from 41.4 to
-// 39.7 ms; the adapted classes move by -4% .. +2%); the uniform coupled
-// classes, whose two halves and two step forms need more, to 72 (1-D) and 80
-// (2-D): at 64 they spilled 112 and 172 B a lane (4e5 pairs x 200 fine steps,
-// 2-D Levy 532 -> 511 us, its general form 607 -> 576; 1-D Merton 332 -> 323);
-// the generic class, whose cases' register needs go up to ~250 VGPRs for the 4-D
-// two-driver family, to 128 (4 wavefronts; a few of its cases spill a
-// little) instead of running at 2 per SIMD.
+// Wavefronts per SIMD.  The dedicated class kernels hold both step forms (the
+// adapted ones the jump queue) and need up to 70 VGPRs, the uniform coupled ones
+// 79 (1-D) and 92 (2-D); they are held to what 7, 6 and 5 wavefronts leave, so
+// none spills.  7 is also what a launch of 7 workgroups of 4 wavefronts per CU,
+// the default, keeps resident.  At 8, 7 and 6 they spilled up to 31 VGPRs
+// (4e5 paths x 96 steps: 1-D Merton pairs 109 -> 105 us, 2-D Levy clock of mixed
+// coefficients 145 -> 135, of constant ones 121 -> 130, the adapted 2-D Levy
+// 136 -> 131; rounds of 16 mixed requests 0-4% less).  The generic class, whose cases' register needs
+// go up to ~250 VGPRs for the 4-D two-driver family, is held to 128 (4
+// wavefronts; a few of its cases spill a little) instead of running at 2.
 constexpr int batch_waves(int cls) {
   if (cls == SDEMC_CLASS_GENERIC) return 4;
-  if (cls == SDEMC_CLASS_DIAG1 + 1) return 7;
-  if (cls == SDEMC_CLASS_INDEP2 + 1) return 6;
-  return 8;
+  if (cls == SDEMC_CLASS_DIAG1 + 1) return 6;
+  if (cls == SDEMC_CLASS_INDEP2 + 1) return 5;
+  return 7;
 }
 
 // Persistent tile kernel of one class group.  hdr = {first segment,

@@ -130,12 +130,12 @@ __device__ __forceinline__ void normals6(const U4& w, float* z) {
   const uint32_t wp[3] = {w.x, w.y, w.z};
 #pragma unroll
   for (int p = 0; p < 3; ++p) {
-    // 1 + a as float bits: 0x3F800000 | (w_p mod 2^9) << 14 | (w3 field) << 4,
-    // in two shifts, an and-or (1.0f is an inline constant) and a bit select
-    const uint32_t field = p == 0 ? w.w << 4 : w.w >> (10 * p - 4);
-    uint32_t lo, bits;
-    asm("v_and_or_b32 %0, %1, %2, 1.0" : "=v"(lo) : "v"(field), "s"(0x3FF0u));
-    asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(bits) : "s"(0x007FC000u), "v"(wp[p] << 14), "v"(lo));
+    // 1 + a as float bits: 0x3F800000 | (w_p mod 2^9) << 14 | (w3 field) << 4.
+    // Left to the compiler: written as and-or and bit-select instructions by
+    // hand, the angles were formed early and held, 4 to 8 registers more in the
+    // step loops without a gain in any (320 launch shapes: 0.4% slower on average)
+    const uint32_t lo = (((w.w >> (10 * p)) & 0x3FFu) << 4) | 0x3F800000u;
+    const uint32_t bits = ((wp[p] << 14) & 0x007FC000u) | lo;
     box_muller_ua(u01_open(wp[p]), __uint_as_float(bits), z[2 * p], z[2 * p + 1]);
   }
 }

@@ -1,0 +1,26 @@
+"""What the built kernels take of the register file: the occupancies their
+launch rules count on, and no spills where every loop turn would pay for them
+(no GPU; the built library's own metadata)."""
+import os
+
+import pytest
+
+from sde_mc_amd import build
+from tests import kernel_notes
+
+if not os.path.exists(build.lib_path()):
+    pytest.skip('library not built', allow_module_level=True)
+
+KERNELS = kernel_notes.kernels()
+
+
+@pytest.mark.parametrize('cls,waves', [(0, 7), (1, 6), (2, 7), (3, 7), (4, 7), (5, 5), (6, 7),
+                                       (7, 7), (8, 7)])
+def test_batched_class_kernels_do_not_spill(cls, waves):
+    for unroll in (1, 2):
+        k = KERNELS.get('k_batch<%d, %d>' % (cls, unroll))
+        assert k is not None or (unroll == 2 and cls not in (0, 4, 8))
+        if k is None:
+            continue
+        assert k.get('.vgpr_spill_count', 0) == 0 and k['.private_segment_fixed_size'] == 0
+        assert kernel_notes.waves_per_simd(k) >= waves
