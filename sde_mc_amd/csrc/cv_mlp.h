@@ -33,19 +33,34 @@ typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 constexpr int CV_BLOCK_WORDS = 512;  // one operand fragment: 64 lanes x 8 bf16
 constexpr int CV_MAX_THREADS = 512;
 
-// Wavefronts per workgroup.  The workgroup's wavefronts share one LDS copy of
-// the weights (22 KB for a network of three hidden layers): workgroups of eight
-// leave room for the sixteen wavefronts a CU that the registers allow where
-// workgroups of four with both networks fit three.  That pays while the
-// launch fits the chip at once (2^18 Merton paths x 300 adapted steps with an f
-// and a g: 2782 -> 2613 us); over several rounds the matrix cores are busy
-// either way and the smaller workgroups hand over sooner (2^20 x 1000: 28.6 ms
-// with four, 29.4 with eight).  A launch of few chunks takes smaller ones,
-// so that it reaches all 256 CUs.
-inline int cv_waves_per_block(int64_t nchunks) {
-  int w = nchunks <= 256 * 16 ? 8 : 4;
-  while (w > 1 && nchunks < 256 * (int64_t)w) w >>= 1;
-  return w;
+// Wavefronts per workgroup: four, or eight where that lets more wavefronts lie on
+// a CU.  The workgroup's wavefronts share one LDS copy of the weights (22 KB for a
+// network of three hidden layers), so with both networks of the 1-D Merton
+// kernel (128 VGPRs) three workgroups of four fit and two of eight: 12 wavefronts
+// a CU against 16 (2^18 paths x 60 adapted steps 508 -> 478 us, 2^20 1815 -> 1769).
+// The wider models' kernels (129 to 159 VGPRs) hold one workgroup of eight, and at
+// eight take 2-10% longer; with one network both sizes fit 16 wavefronts and four
+// hands over sooner.  A launch that does not fill the CUs with workgroups of
+// eight takes four (1e4 paths: 1.3 times as long with eight, the same with two
+// or one).
+inline int cv_waves_per_block(int64_t nchunks, int vgprs, size_t lds) {
+  constexpr int CUS = 256, SIMDS = 4;
+  constexpr size_t LDS = 160 << 10;
+  auto resident = [&](int wpb) {
+    const int by_regs = SIMDS * (512 / ((vgprs + 7) / 8 * 8)) / wpb;
+    const int by_lds = lds > 0 ? (int)(LDS / lds) : by_regs;
+    return wpb * (by_regs < by_lds ? by_regs : by_lds);
+  };
+  return nchunks >= CUS * 8 && resident(8) > resident(4) ? 8 : 4;
+}
+
+// Vector registers of a kernel, asked for once by each launcher (all of them when
+// the runtime does not say: workgroups of four then).
+inline int cv_kernel_vgprs(const void* kernel) {
+  hipFuncAttributes a;
+  if (hipFuncGetAttributes(&a, kernel) == hipSuccess && a.numRegs > 0) return a.numRegs;
+  (void)hipGetLastError();
+  return 512;
 }
 
 __host__ __device__ constexpr int cv_blocks(int hidden) { return 8 * hidden - 2; }
@@ -429,10 +444,11 @@ struct CvLaunch {
 
 template <int D, int FAM>
 int launch_cv_uniform_d(const KJob& job, const CvLaunch& a, int64_t nchunks) {
-  const int wpb = cv_waves_per_block(nchunks);
+  static const int vgprs = cv_kernel_vgprs((const void*)k_cv_uniform<D, FAM>);
+  const size_t lds = (size_t)cv_words(a.f_hidden) * 2;
+  const int wpb = cv_waves_per_block(nchunks, vgprs, lds);
   const int64_t blocks = (nchunks + wpb - 1) / wpb;
   if (blocks <= 0 || blocks > 0x7fffffffLL) return SDEMC_ERR_ARG;
-  const size_t lds = (size_t)cv_words(a.f_hidden) * 2;
   hipLaunchKernelGGL((k_cv_uniform<D, FAM>), dim3((unsigned)blocks), dim3(WAVE * wpb), lds,
                      a.stream, job, a.fw, a.f_hidden, a.rate, a.cv_steps, a.partials, a.cflags,
                      a.gamma, nchunks);
@@ -441,10 +457,11 @@ int launch_cv_uniform_d(const KJob& job, const CvLaunch& a, int64_t nchunks) {
 
 template <int D, int FAM>
 int launch_cv_adapted_d(const KJob& job, const CvLaunch& a, int64_t nchunks) {
-  const int wpb = cv_waves_per_block(nchunks);
+  static const int vgprs = cv_kernel_vgprs((const void*)k_cv_adapted<D, FAM>);
+  const size_t lds = (size_t)(cv_words(a.f_hidden) + cv_words(a.g_hidden)) * 2;
+  const int wpb = cv_waves_per_block(nchunks, vgprs, lds);
   const int64_t blocks = (nchunks + wpb - 1) / wpb;
   if (blocks <= 0 || blocks > 0x7fffffffLL) return SDEMC_ERR_ARG;
-  const size_t lds = (size_t)(cv_words(a.f_hidden) + cv_words(a.g_hidden)) * 2;
   hipLaunchKernelGGL((k_cv_adapted<D, FAM>), dim3((unsigned)blocks), dim3(WAVE * wpb), lds,
                      a.stream, job, a.fw, a.f_hidden, a.gw, a.g_hidden, a.rate, a.comp,
                      a.cv_steps, a.partials, a.cflags, a.gamma, nchunks);

@@ -186,6 +186,21 @@ struct BmStream {
   __device__ __forceinline__ void normals(uint32_t b, float* z) const { normals6(block(b), z); }
 };
 
+// The same blocks, each drawn from the beginning, for kernels whose occupancy
+// the held products cost more than the five operations a block.
+struct BmPlain {
+  uint32_t k0, k1, plo, phi;
+  __device__ __forceinline__ void init(uint32_t key0, uint32_t key1, uint32_t lo, uint32_t hi) {
+    k0 = key0;
+    k1 = key1;
+    plo = lo;
+    phi = hi;
+  }
+  __device__ __forceinline__ void normals(uint32_t b, float* z) const {
+    normals6(philox4x32_10(b, STREAM_BM, plo, phi, k0, k1), z);
+  }
+};
+
 // Steps (or adapted-grid rows) whose K normals each are drawn together as
 // whole blocks: 4 when 4K normals fill whole blocks (K = 3), else 6.
 __host__ __device__ constexpr int group_steps(int K) { return (4 * K) % NORMALS_PER_BLOCK == 0 ? 4 : 6; }
@@ -241,9 +256,11 @@ __device__ __forceinline__ float ln_unit(uint32_t w) {
 
 // Normal number i of one path (i = step * K + k): normal i mod 6 of Philox
 // block i / 6 on the Brownian stream (normals6).  The last block is cached,
-// so sequential reads cost one Philox block per 6 normals.
+// so sequential reads cost one Philox block per 6 normals.  The control-variate
+// kernels read it beside their accumulators: with the held products the 1-D
+// Merton one took 161 VGPRs, 3 wavefronts per SIMD, instead of 128 and 4.
 struct NormalStream {
-  BmStream bm;
+  BmPlain bm;
   uint32_t blk;
   float z[NORMALS_PER_BLOCK];
   __device__ __forceinline__ void init(uint32_t key0, uint32_t key1, uint64_t path) {

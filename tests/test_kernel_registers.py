@@ -24,3 +24,11 @@ def test_batched_class_kernels_do_not_spill(cls, waves):
             continue
         assert k.get('.vgpr_spill_count', 0) == 0 and k['.private_segment_fixed_size'] == 0
         assert kernel_notes.waves_per_simd(k) >= waves
+
+
+def test_control_variate_kernels_keep_their_wavefronts():
+    # the 1-D Merton kernel's workgroups of eight rest on four wavefronts per SIMD
+    assert kernel_notes.waves_per_simd(KERNELS['k_cv_adapted<1, 0>']) >= 4
+    for name, k in KERNELS.items():
+        if name.startswith('k_cv_adapted<') or name.startswith('k_cv_uniform<'):
+            assert kernel_notes.waves_per_simd(k) >= (4 if 'uniform' in name else 3), name
