@@ -1932,7 +1932,6 @@ __device__ __forceinline__ bool isclose32(float tau, float t) {
 // draws happen.
 template <int D, int FAM>
 struct AdaptRngSrc {
-  static constexpr bool SORTED = true;  // jump times never decrease
   NormalStream ns;
   JumpClock jc;  // the last jump drawn
   uint32_t plo, phi, k0, k1;
@@ -1996,8 +1995,7 @@ struct AdaptRngSrc {
 // queue leaves almost none.
 template <int D, int FAM>
 struct AdaptQueueSrc {
-  static constexpr bool SORTED = true;  // jump times never decrease
-  JumpClock jc;                         // the last jump drawn
+  JumpClock jc;  // the last jump drawn
   uint32_t plo, phi, k0, k1, lane;
   BmStream bm;
   uint32_t head;
@@ -2089,7 +2087,6 @@ struct AdaptQueueSrc {
 
 template <int D, int FAM>
 struct AdaptFixedSrc {
-  static constexpr bool SORTED = false;
   const sdemc_fixed_in* in;
   int64_t p, P;
   int32_t jn;
@@ -2178,9 +2175,9 @@ struct HeldCoef {
 //
 // A row's clock is kept to two operations and one compare.  The step
 // dt = min(h, T - t, tau - t) is min(h, lim - t) with lim = min(tau, T): fp32
-// subtraction is monotone, and a nominal step cut at T stays cut at every later
-// row, so this is the reference's running h (solvers.py:187-191) bit for bit;
-// caller-supplied jump times need not be sorted and keep the running form.
+// subtraction is monotone, the drawn jump times never decrease and a nominal
+// step cut at T stays cut at every later row, so this is the reference's running
+// h (solvers.py:187-191) bit for bit.
 // A row ends in an event -- a jump, the horizon, the step limit -- only if t
 // reaches ev = min(tau - margin, T), margin above the tolerance of the jump
 // test; lim and ev change only in events.  A finished lane keeps its state in
@@ -2241,12 +2238,7 @@ __device__ int32_t path_adapted(const KJob& j, SRC& src, bool lane_valid, int64_
       float dt;
       {
 #pragma clang fp contract(off)
-        if constexpr (SRC::SORTED) {
-          dt = min_num(h, lim - t);
-        } else {
-          h = fminf(h, fmaxf(T32 - t, 0.0f));
-          dt = fminf(h, lim - t);
-        }
+        dt = min_num(h, lim - t);
       }
       const float sq = __builtin_amdgcn_sqrtf(dt);
       float zz[K];
@@ -2354,6 +2346,74 @@ __device__ int32_t path_adapted(const KJob& j, SRC& src, bool lane_valid, int64_
       if (st.normals) {
 #pragma unroll
         for (int k = 0; k < KN; ++k) st.normals[((int64_t)r * KN + k) * st.P + p] = 0.0f;
+      }
+    }
+  }
+  return steps;
+}
+
+// Single level on the adapted grid from caller-supplied inputs.  The jump times
+// need not be sorted, so the step keeps the reference's running h
+// (solvers.py:187-191) and every row tests for its jump: with the rows' event
+// test of path_adapted instead, 10^4 Merton paths x 48 steps took 23.0 us instead of 20.2
+// (2e5: 36.3, 34.6).
+template <int D, int FAM>
+__device__ int32_t path_adapted_fixed(const KJob& j, AdaptFixedSrc<D, FAM>& src, bool lane_valid,
+                                      float (&x)[D], int& overflow) {
+  constexpr int K = NK<D, FAM>::K;
+  constexpr int G = group_steps(K);
+  const KModel& f = j.m;
+  const float T32 = (float)j.T;
+  const int32_t max_steps = j.max_steps;
+  float h = j.h;
+  float t = 0.0f;
+#pragma unroll
+  for (int i = 0; i < D; ++i) x[i] = f.x0[i];
+  float tau = lane_valid ? src.next_time() : 0.0f;
+  bool active = lane_valid && (t < T32);
+  int32_t steps = 0;
+  overflow = 0;
+  for (uint32_t row0 = 0; __any(active); row0 += G) {
+    float zq[G * K];
+    src.rows(row0, active, zq);
+#pragma unroll
+    for (int q = 0; q < G; ++q) {
+      if (active && steps >= max_steps) {
+        overflow = 1;
+        active = false;
+      }
+      if (active) {
+        float dt;
+        {
+#pragma clang fp contract(off)
+          h = fminf(h, fmaxf(T32 - t, 0.0f));
+          dt = fminf(h, tau - t);
+        }
+        const float sq = __builtin_amdgcn_sqrtf(dt);
+        float dW[D], dB[D], xo[D];
+        correlate<D, FAM>(f, &zq[q * K], sq, dW, dB);
+#pragma unroll
+        for (int i = 0; i < D; ++i) xo[i] = x[i];
+        euler<D, FAM>(f, x, dt, dW, dB);
+        {
+#pragma clang fp contract(off)
+          t = t + dt;
+        }
+        ++steps;
+        if (isclose32(tau, t)) {
+          const float J = src.mark(f, true);
+          if (f.exact) {
+            float y[D];
+#pragma unroll
+            for (int i = 0; i < D; ++i) y[i] = x[i];
+            add_jump(f, x, y, J);
+          } else {
+            add_jump(f, x, xo, J);
+          }
+          src.advance(f, true);
+          tau = src.next_time();
+        }
+        active = t < T32;
       }
     }
   }

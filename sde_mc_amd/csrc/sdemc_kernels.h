@@ -240,7 +240,6 @@ __global__ __launch_bounds__(256) void k_fixed(const KJob job, const sdemc_fixed
   const int64_t p = chunk * WAVE + lane;
   const bool valid = p < P;
   const KPayoff& pf = job.pay;
-  StoreCtx st{};
   float v = 0.0f;
   int ovf = 0, bad = 0;
   int32_t nsteps = job.steps;
@@ -251,7 +250,7 @@ __global__ __launch_bounds__(256) void k_fixed(const KJob job, const sdemc_fixed
     } else {
       AdaptFixedSrc<D, FAM> src;
       src.init(in, p, P);
-      nsteps = path_adapted<D, FAM, false>(job, src, valid, p, x, ovf, st);
+      nsteps = path_adapted_fixed<D, FAM>(job, src, valid, x, ovf);
     }
     if (valid) {
       v = payoff_raw<D>(pf, x) * pf.disc;

@@ -32,3 +32,9 @@ def test_control_variate_kernels_keep_their_wavefronts():
     for name, k in KERNELS.items():
         if name.startswith('k_cv_adapted<') or name.startswith('k_cv_uniform<'):
             assert kernel_notes.waves_per_simd(k) >= (4 if 'uniform' in name else 3), name
+
+
+def test_fixed_increment_adapted_kernels_hold_no_event_state():
+    # the drawn path's event test in this kernel took 38 registers and 14% more time
+    assert KERNELS['k_fixed<1, 0, 1, false>']['.vgpr_count'] <= 34
+    assert KERNELS['k_fixed<1, 1, 1, false>']['.vgpr_count'] <= 40
