@@ -200,6 +200,8 @@ struct BmPlain {
     normals6(philox4x32_10(b, STREAM_BM, plo, phi, k0, k1), z);
   }
 };
+template <bool HELD>
+using BmBlocks = std::conditional_t<HELD, BmStream, BmPlain>;
 
 // Steps (or adapted-grid rows) whose K normals each are drawn together as
 // whole blocks: 4 when 4K normals fill whole blocks (K = 3), else 6.
@@ -1385,7 +1387,11 @@ __device__ void path_uniform_rng_form(const KJob& j, const PathCtx& c, bool lane
   const float sq = j.sqh;
   const uint32_t plo = (uint32_t)c.path, phi = (uint32_t)(c.path >> 32);
   constexpr bool pois = POIS;
-  BmStream bm;
+  // products held along the path but where registers are short: a coupled
+  // pair's general loop, and storing kernels, whose addresses take theirs (4-D
+  // Merton 71 VGPRs, 92 with them and the loop below in full groups: 7 -> 5
+  // wavefronts per SIMD, 2e5 paths x 96 steps 185 -> 219 us)
+  BmBlocks<!STORE && !(COUPLED && UF == UFORM_ANY)> bm;
   bm.init(c.k0, c.k1, plo, phi);
   // the common forms' jump coefficients: the exponential Levy's are constant,
   // the proportional ones are not (takes_common_form asks for both)
@@ -1495,11 +1501,7 @@ __device__ void path_uniform_rng_form(const KJob& j, const PathCtx& c, bool lane
     const uint32_t b0 = (uint32_t)n0 * (uint32_t)K / (uint32_t)NORMALS_PER_BLOCK;
 #pragma unroll
     for (int b = 0; b < G * K / NORMALS_PER_BLOCK; ++b)
-      // (a coupled pair's general loop is short of registers: no products held)
-      if constexpr (COUPLED && UF == UFORM_ANY)
-        normals6(philox4x32_10(b0 + b, STREAM_BM, plo, phi, c.k0, c.k1), &z[NORMALS_PER_BLOCK * b]);
-      else
-        bm.normals(b0 + b, &z[NORMALS_PER_BLOCK * b]);
+      bm.normals(b0 + b, &z[NORMALS_PER_BLOCK * b]);
 #pragma unroll
     for (int s = 0; s < G; ++s) {
       const int32_t n = n0 + s;
@@ -1511,9 +1513,12 @@ __device__ void path_uniform_rng_form(const KJob& j, const PathCtx& c, bool lane
         for (int i = 0; i < D; ++i) xo[i] = x[i];
         uniform_step<D, FAM, UF>(j, x, &z[s * K], fine, UF == UFORM_PROP ? uA : j.uA);
         float jsum = 0.0f;
-        // rare enough (and long) to be laid out of line: steps without a jump
-        // run straight on
-        if (!pois && __builtin_expect(__any(n == hk), 0)) {
+        // a common form's step without a jump runs straight on, the jumps laid
+        // out of line; the general form's tests its lanes in line (out of line
+        // its small launches, whose wavefronts meet a jump at most steps, take
+        // two branches more a step: 1e4 3-D Merton paths of mixed coefficients
+        // x 96 steps 52.4 us against 49.3)
+        if (!pois && (UF == UFORM_ANY ? n == hk : (bool)__builtin_expect(__any(n == hk), 0))) {
           while (n == hk) {
             const float J = cq->J[qh][lane];
             if (additive) {  // fma(j1, y, j0) = j0 exactly: add_jump's bits, one operation
@@ -1647,24 +1652,31 @@ __device__ void path_uniform_rng_form(const KJob& j, const PathCtx& c, bool lane
       spill = __any(kj < wend);
     }
   };
-  // the general form of larger states keeps the end tests: without them the
-  // compiler holds more values across steps than the wavefronts pay for
-  using Full = std::bool_constant<!(UF == UFORM_ANY && D > (COUPLED ? 1 : 2))>;
+  // the general form of larger states and of storing kernels keeps the end
+  // tests, in one loop: without them the compiler holds more values across
+  // steps than the wavefronts pay for, and a second loop for the last steps
+  // doubles its code (1e4 2-D Merton paths x 96 steps stored 56.7 us against 51.8)
+  constexpr bool FULL = !(UF == UFORM_ANY && (STORE || D > (COUPLED ? 1 : 2)));
+  using Full = std::bool_constant<FULL>;
   int32_t n0 = 0;
-  for (; n0 + G * U <= N; n0 += G * U) {
+  for (; FULL ? n0 + G * U <= N : n0 < N; n0 += G * U) {
     window(n0);
     if (spill) {
 #pragma unroll
-      for (int u = 0; u < U; ++u) group(n0 + G * u, std::true_type{}, Full{});
+      for (int u = 0; u < U; ++u)
+        if (FULL || u == 0 || n0 + G * u < N) group(n0 + G * u, std::true_type{}, Full{});
     } else {
 #pragma unroll
-      for (int u = 0; u < U; ++u) group(n0 + G * u, std::false_type{}, Full{});
+      for (int u = 0; u < U; ++u)
+        if (FULL || u == 0 || n0 + G * u < N) group(n0 + G * u, std::false_type{}, Full{});
     }
   }
-  // the last steps of a grid that is no multiple of the stride
-  for (; n0 < N; n0 += G) {
-    window(n0);
-    group(n0, std::true_type{}, std::false_type{});
+  if constexpr (FULL) {
+    // the last steps of a grid that is no multiple of the stride
+    for (; n0 < N; n0 += G) {
+      window(n0);
+      group(n0, std::true_type{}, std::false_type{});
+    }
   }
 }
 

@@ -38,3 +38,13 @@ def test_fixed_increment_adapted_kernels_hold_no_event_state():
     # the drawn path's event test in this kernel took 38 registers and 14% more time
     assert KERNELS['k_fixed<1, 0, 1, false>']['.vgpr_count'] <= 34
     assert KERNELS['k_fixed<1, 1, 1, false>']['.vgpr_count'] <= 40
+
+
+@pytest.mark.parametrize('family', ['0', '1'])
+@pytest.mark.parametrize('pois', ['false', 'true'])
+def test_storing_uniform_kernels_keep_their_wavefronts(family, pois):
+    # up to 4 components, beside the addresses of three stored arrays
+    for dim, waves in ((1, 8), (2, 8), (3, 7), (4, 6)):
+        k = KERNELS['k_rng<%d, %s, 0, false, true, %s, -1>' % (dim, family, pois)]
+        assert k['.private_segment_fixed_size'] == 0
+        assert kernel_notes.waves_per_simd(k) >= waves
