@@ -245,7 +245,7 @@ __device__ __forceinline__ float cv_dot(const float (&fo)[8], const float (&dW)[
 }
 
 // Uniform grid without jumps (apply_diffusion_control_variate): steps as in
-// path_uniform_rng, t_n = n h.
+// path_uniform_rng_form, t_n = n h.
 template <int D, int FAM>
 __global__ __launch_bounds__(CV_MAX_THREADS) void k_cv_uniform(const KJob job, const uint16_t* fw,
                                                     int32_t f_hidden, float rate,

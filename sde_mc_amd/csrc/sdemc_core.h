@@ -219,8 +219,10 @@ __device__ __forceinline__ float fast_ln(float v) {
 
 // n / d correctly rounded for operands whose quotient and residuals need no
 // scaling (d within a few binades of 1, |n| <= d, n zero or not tiny): the
-// reciprocal refined once and the quotient twice, without the scaling and
-// special cases of __fdiv_rn; the same bits with three instructions fewer.
+// reciprocal refined once and the quotient twice by their residuals (Markstein,
+// IBM J. Res. Dev. 34, 1990), the steps of the AMDGPU back end's correctly rounded
+// quotient (LLVM, open source) without its scaling and special cases; the same
+// bits as __fdiv_rn with three instructions fewer.
 __device__ __forceinline__ float div_rn_unscaled(float n, float d) {
   float r = __builtin_amdgcn_rcpf(d);
   r = __fmaf_rn(__fmaf_rn(-d, r, 1.0f), r, r);
@@ -665,8 +667,10 @@ __device__ __forceinline__ float payoff_raw(const KPayoff& p, const float (&x)[D
   return v;
 }
 
-// sqrt(x) correctly rounded, x >= 2^-96 or 0: the hardware root (within one
-// unit) and its two neighbours, told apart by their exact residuals.
+// sqrt(x) correctly rounded, x >= 2^-96 or 0 (within one unit below): the hardware
+// root (within one unit) and its two neighbours, told apart by their exact
+// residuals, as the AMDGPU back end's correctly rounded root does (LLVM, open
+// source), without its scaling of small x.
 __device__ __forceinline__ float sqrt_rn_unscaled(float x) {
   float s = __builtin_amdgcn_sqrtf(x);
   const float lo = __uint_as_float(__float_as_uint(s) - 1u);
@@ -2067,19 +2071,19 @@ struct AdaptQueueSrc {
     for (int b = 0; b < G * K / NORMALS_PER_BLOCK; ++b)
       bm.normals(b0 + b, &zq[NORMALS_PER_BLOCK * b]);
   }
-  __device__ __forceinline__ float next_time(bool = true) const {
+  __device__ __forceinline__ float next_time() const {
     return __int_as_float(cq->k[head % CLOCK_JQ][lane]);
   }
-  __device__ __forceinline__ float mark(const KModel&, bool) const {
+  __device__ __forceinline__ float mark(const KModel&) const {
     return cq->J[head % CLOCK_JQ][lane];
   }
-  // past the pending jump where `hit`; next_time() is then the one after
-  __device__ __forceinline__ void advance(const KModel& f, bool hit) {
-    const bool dry = hit && head == jc.j;
+  // past the pending jump; next_time() is then the one after
+  __device__ __forceinline__ void advance(const KModel& f) {
+    const bool dry = head == jc.j;
     if (__builtin_expect(__any(dry), 0)) {
       if (dry) draw_next(f);
     }
-    head += hit ? 1u : 0u;
+    ++head;
   }
   // whole wavefront: the jumps of every live lane up to time `until`, and the
   // one after, as far as its queue holds them
@@ -2123,13 +2127,13 @@ struct AdaptFixedSrc {
 #pragma unroll
       for (int k = 0; k < K; ++k) zq[q * K + k] = live ? z(row0 + (uint32_t)q, k) : 0.0f;
   }
-  __device__ __forceinline__ float next_time(bool hit = true) const {
-    return hit && jn < in->max_jumps ? in->jump_time_dev[(int64_t)jn * P + p] : __builtin_inff();
+  __device__ __forceinline__ float next_time() const {
+    return jn < in->max_jumps ? in->jump_time_dev[(int64_t)jn * P + p] : __builtin_inff();
   }
-  __device__ __forceinline__ float mark(const KModel&, bool hit) const {
-    return hit && jn < in->max_jumps ? in->jump_size_dev[(int64_t)jn * P + p] : 0.0f;
+  __device__ __forceinline__ float mark(const KModel&) const {
+    return jn < in->max_jumps ? in->jump_size_dev[(int64_t)jn * P + p] : 0.0f;
   }
-  __device__ __forceinline__ void advance(const KModel&, bool hit) { jn += hit ? 1 : 0; }
+  __device__ __forceinline__ void advance(const KModel&) { ++jn; }
   __device__ __forceinline__ void fill(const KModel&, bool, float) {}
 };
 
@@ -2293,15 +2297,15 @@ __device__ int32_t path_adapted(const KJob& j, SRC& src, bool lane_valid, int64_
         // one costs a wavefront that has its SIMD to itself about as long as
         // ten instructions
         if (t >= ev && isclose32(tau, t)) {
-          const float J = src.mark(f, true);
+          const float J = src.mark(f);
 #pragma unroll
           for (int i = 0; i < D; ++i) {
             const float y = f.exact ? x[i] : xo[i];  // add_jump
             x[i] = __fmaf_rn(__fmaf_rn(f.j1[i], y, f.j0[i]), J, x[i]);
           }
           Jap = J;
-          src.advance(f, true);
-          tau = src.next_time(true);
+          src.advance(f);
+          tau = src.next_time();
           lim = fminf(tau, T32);
           ev = last ? -__builtin_inff() : fminf(tau - margin, T32);
         }
@@ -2413,7 +2417,7 @@ __device__ int32_t path_adapted_fixed(const KJob& j, AdaptFixedSrc<D, FAM>& src,
         }
         ++steps;
         if (isclose32(tau, t)) {
-          const float J = src.mark(f, true);
+          const float J = src.mark(f);
           if (f.exact) {
             float y[D];
 #pragma unroll
@@ -2422,7 +2426,7 @@ __device__ int32_t path_adapted_fixed(const KJob& j, AdaptFixedSrc<D, FAM>& src,
           } else {
             add_jump(f, x, xo, J);
           }
-          src.advance(f, true);
+          src.advance(f);
           tau = src.next_time();
         }
         active = t < T32;
@@ -2542,7 +2546,7 @@ __device__ int32_t path_adapted_coupled(const KJob& j, SRC& src, bool lane_valid
           }
           const bool hit = isclose32(tau, tf);
           if (hit) {
-            const float J = src.mark(f, true);
+            const float J = src.mark(f);
             if (f.exact) {
               float y[D];
 #pragma unroll
@@ -2555,7 +2559,7 @@ __device__ int32_t path_adapted_coupled(const KJob& j, SRC& src, bool lane_valid
               add_jump(f, xf, xfo, J);
               add_jump(f, xc, xco, J);
             }
-            src.advance(f, true);
+            src.advance(f);
             tau = src.next_time();
           }
           if (!(tf < T32)) {
