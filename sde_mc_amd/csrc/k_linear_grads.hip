@@ -7,11 +7,9 @@
 // dimension: each wavefront multiplies its own rows on
 // v_mfma_f32_32x32x2_f32 (fp32 throughout), reading both operands straight
 // from memory as the instruction takes them -- 32 consecutive columns of two
-// rows, whole lines -- with no staging.  Partial results are summed in a fixed
-// order: wavefronts of a workgroup in LDS, workgroups by k_linear_grads_sum.
-// db's sums run in fp64 beside the product (hidden by it): as a further fp32
-// column of it they were off by 1.3 to 1.8 times the library's sum, which adds
-// in a tree; dW is off by 0.03 to 0.1 of u sum |terms|, the library's by 0.1 to 0.5.
+// rows, whole lines -- with no staging; the 1 in column n_in of X makes db a
+// column of the same product.  Partial results are summed in a fixed order:
+// wavefronts of a workgroup in LDS, workgroups by k_linear_grads_sum.
 // Bound by the operands' reads (20 MB, 4 us at the copy rate) and two launches:
 // both gradients of 48000 x 50 x 50 take 16 us, launches included, against 128 us
 // for the library's product (tiles of the result without a split of the inner
@@ -45,28 +43,18 @@ static inline LgShape lg_shape(int64_t rows, int32_t n_in, int32_t n_out) {
   return s;
 }
 
-constexpr int LG_COLS = 64;  // columns of db's partials, each two floats: value and rest
-
-__device__ __forceinline__ void lg_split(double v, float* out) {
-  const float hi = (float)v;
-  out[0] = hi;
-  out[1] = isfinite(hi) ? (float)(v - (double)hi) : 0.0f;
-}
-
-// MT, NT: 32-wide tiles over the columns of dY and X.  partials: a tile set per
-// workgroup; db_partials: LG_COLS columns per workgroup.
+// MT, NT: 32-wide tiles over the columns of dY and over those of X and the 1.
 template <int MT, int NT>
 __global__ __launch_bounds__(WAVE * LG_WAVES) void k_linear_grads(
     const float* __restrict__ x, const float* __restrict__ dy, const LgShape s,
-    float* __restrict__ partials, float* __restrict__ db_partials) {
-  __shared__ __align__(16) float tile[LG_WAVES][MT * NT * 16 * WAVE];
+    float* __restrict__ partials) {
+  __shared__ float tile[LG_WAVES][MT * NT * 16 * WAVE];
   const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
   const int col = lane & 31, half = lane >> 5;
   const int64_t r0 = ((int64_t)blockIdx.x * LG_WAVES + wave) * s.rows_per_wave;
   int64_t r1 = r0 + s.rows_per_wave;
   if (r1 > s.rows) r1 = s.rows;
   lg_f32x16 acc[MT][NT];
-  double sum[MT] = {};  // of this lane's column of dY over its rows
 #pragma unroll
   for (int m = 0; m < MT; ++m)
 #pragma unroll
@@ -85,18 +73,16 @@ __global__ __launch_bounds__(WAVE * LG_WAVES) void k_linear_grads(
 #pragma unroll
       for (int n = 0; n < NT; ++n) {
         const int c = 32 * n + col;
-        b[t][n] = in && c < s.n_in ? x[row * s.n_in + c] : 0.0f;
+        b[t][n] = in && c < s.n_in ? x[row * s.n_in + c] : (c == s.n_in ? 1.0f : 0.0f);
       }
     }
 #pragma unroll
     for (int t = 0; t < LG_STEPS; ++t)
 #pragma unroll
-      for (int m = 0; m < MT; ++m) {
-        sum[m] += (double)a[t][m];
+      for (int m = 0; m < MT; ++m)
 #pragma unroll
         for (int n = 0; n < NT; ++n)
           acc[m][n] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[t][m], b[t][n], acc[m][n], 0, 0, 0);
-      }
   }
 #pragma unroll
   for (int m = 0; m < MT; ++m)
@@ -112,48 +98,19 @@ __global__ __launch_bounds__(WAVE * LG_WAVES) void k_linear_grads(
     for (int w = 1; w < LG_WAVES; ++w) v += tile[w][e];
     partials[(int64_t)blockIdx.x * SIZE + e] = v;
   }
-  __syncthreads();
-  double* const sums = reinterpret_cast<double*>(&tile[0][0]);
-#pragma unroll
-  for (int m = 0; m < MT; ++m) sums[(wave * 2 + half) * LG_COLS + 32 * m + col] = sum[m];
-  __syncthreads();
-  if (threadIdx.x < 32 * MT) {
-    double v = 0.0;
-#pragma unroll
-    for (int q = 0; q < 2 * LG_WAVES; ++q) v += sums[q * LG_COLS + threadIdx.x];
-    lg_split(v, db_partials + 2 * ((int64_t)blockIdx.x * LG_COLS + threadIdx.x));
-  }
 }
 
 // Sum of the workgroups' partials: workgroup e / 64 takes the 64 elements of one
 // accumulator of one tile (lane l: row 8 (q / 4) + 4 (l / 32) + q % 4, column
-// l % 32), its 16 wavefronts a sixteenth of the partials each; the workgroup past
-// the last accumulator takes db's 64 columns.
+// l % 32), its 16 wavefronts a sixteenth of the partials each.
 __global__ __launch_bounds__(1024) void k_linear_grads_sum(const float* __restrict__ partials,
-                                                           const float* __restrict__ db_partials,
                                                            int32_t blocks, int32_t size,
                                                            int32_t nt, int32_t n_in, int32_t n_out,
                                                            float* __restrict__ dw,
                                                            float* __restrict__ db) {
   __shared__ float part[16][WAVE];
-  __shared__ double dpart[16][WAVE];
   const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
   const int e = blockIdx.x * WAVE + lane;
-  if (e >= size) {  // db's workgroup
-    double v = 0.0;
-    if (lane < n_out)
-      for (int b = wave; b < blocks; b += 16) {
-        const float* p = db_partials + 2 * ((int64_t)b * LG_COLS + lane);
-        v += (double)p[0] + (double)p[1];
-      }
-    dpart[wave][lane] = v;
-    __syncthreads();
-    if (wave != 0 || lane >= n_out) return;
-#pragma unroll
-    for (int w = 1; w < 16; ++w) v += dpart[w][lane];
-    db[lane] = (float)v;
-    return;
-  }
   float v = 0.0f;
   for (int b = wave; b < blocks; b += 16) v += partials[(int64_t)b * size + e];
   part[wave][lane] = v;
@@ -164,7 +121,9 @@ __global__ __launch_bounds__(1024) void k_linear_grads_sum(const float* __restri
   const int q = blockIdx.x & 15, t = blockIdx.x >> 4;
   const int o = 32 * (t / nt) + 8 * (q / 4) + 4 * (lane >> 5) + q % 4;
   const int i = 32 * (t % nt) + (lane & 31);
-  if (o < n_out && i < n_in) dw[(int64_t)o * n_in + i] = v;
+  if (o >= n_out) return;
+  if (i < n_in) dw[(int64_t)o * n_in + i] = v;
+  else if (i == n_in && db) db[o] = v;
 }
 
 }  // namespace sdemc
@@ -175,8 +134,8 @@ extern "C" {
 
 size_t sdemc_linear_grads_floats(int64_t rows, int32_t n_in, int32_t n_out) {
   if (rows < 1 || n_in < 1 || n_in > 63 || n_out < 1 || n_out > 64) return 0;
-  const int mt = (n_out + 31) / 32, nt = (n_in + 31) / 32;
-  return (size_t)lg_shape(rows, n_in, n_out).blocks * (size_t)(mt * nt * 16 * WAVE + 2 * LG_COLS);
+  const int mt = (n_out + 31) / 32, nt = (n_in + 32) / 32;
+  return (size_t)lg_shape(rows, n_in, n_out).blocks * (size_t)(mt * nt * 16 * WAVE);
 }
 
 int sdemc_linear_grads(const float* x_dev, const float* dy_dev, int64_t rows, int32_t n_in,
@@ -187,20 +146,18 @@ int sdemc_linear_grads(const float* x_dev, const float* dy_dev, int64_t rows, in
   if (!x_dev || !dy_dev || !dw_dev || !workspace_dev) return SDEMC_ERR_ARG;
   if (workspace_floats < need) return SDEMC_ERR_WORKSPACE;
   const LgShape s = lg_shape(rows, n_in, n_out);
-  const int mt = (n_out + 31) / 32, nt = (n_in + 31) / 32;
+  const int mt = (n_out + 31) / 32, nt = (n_in + 32) / 32;
   const dim3 g((unsigned)s.blocks), b(WAVE * LG_WAVES);
-  float* const db_partials = workspace_dev + (size_t)s.blocks * (size_t)(mt * nt * 16 * WAVE);
   const hipStream_t st = (hipStream_t)stream;
 #define SDEMC_LG(M, N) \
-  hipLaunchKernelGGL((k_linear_grads<M, N>), g, b, 0, st, x_dev, dy_dev, s, workspace_dev, \
-                     db_partials)
+  hipLaunchKernelGGL((k_linear_grads<M, N>), g, b, 0, st, x_dev, dy_dev, s, workspace_dev)
   if (mt == 1 && nt == 1) SDEMC_LG(1, 1);
   else if (mt == 1) SDEMC_LG(1, 2);
   else if (nt == 1) SDEMC_LG(2, 1);
   else SDEMC_LG(2, 2);
 #undef SDEMC_LG
-  hipLaunchKernelGGL(k_linear_grads_sum, dim3((unsigned)(mt * nt * 16 + (db_dev ? 1 : 0))),
-                     dim3(1024), 0, st, workspace_dev, db_partials, s.blocks, mt * nt * 16 * WAVE, nt, n_in, n_out, dw_dev, db_dev);
+  hipLaunchKernelGGL(k_linear_grads_sum, dim3((unsigned)(mt * nt * 16)), dim3(1024), 0, st,
+                     workspace_dev, s.blocks, mt * nt * 16 * WAVE, nt, n_in, n_out, dw_dev, db_dev);
   return hipGetLastError() == hipSuccess ? SDEMC_OK : SDEMC_ERR_LAUNCH;
 }
 
