@@ -330,7 +330,7 @@ def hbm_read_ceiling(dev, gib=4, reps=5):
 # keyed by the launch shape's chunks per tile: nearly all of it is the chunk
 # partials' writes, which scatter more with one chunk per tile; and the
 # fixed-increment kernel (2^21 x 500).
-TRAFFIC_MIX_ROUND = {1: 9.504e7, 2: 7.103e7}  # tile_chunks -> HBM bytes of one mix round
+TRAFFIC_MIX_ROUND = {1: 8.612e7, 2: 6.206e7}  # tile_chunks -> HBM bytes of one mix round
 TRAFFIC_FIXED = 5.711e9      # HBM bytes of one fixed-increment launch (2^21 x 500)
 # VALU instructions (wavefront-level, SQ_INSTS_VALU summed over the group
 # kernels) of one round of the served mix (128 requests, seed 0) and the fp32
@@ -339,7 +339,7 @@ TRAFFIC_FIXED = 5.711e9      # HBM bytes of one fixed-increment launch (2^21 x 5
 # instruction holds its SIMD for 4 cycles, one per CU-cycle over the 4 SIMDs;
 # the transcendentals overlap the instructions after them, so the issue
 # figure counts the others.
-VALU_INSTR_MIX_ROUND = 2.678e10
+VALU_INSTR_MIX_ROUND = 2.470e10
 VALU_TRANS_MIX_ROUND = 2.031e9
 
 
