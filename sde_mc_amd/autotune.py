@@ -17,7 +17,7 @@ import torch
 from . import _lib as L
 from .batch import BatchRunner, BatchTune, chunks_of, job_class
 
-# A CU has 4 SIMDs and the tile kernels fit 7 or 8 wavefronts per SIMD, so
+# A CU has 4 SIMDs and the tile kernels fit 5 to 7 wavefronts per SIMD, so
 # the shapes swept are workgroups of 2, 4 or 8 wavefronts (128, 256 or 512
 # paths) with 3..8 resident wavefronts per SIMD in all, 1 or 2 chunks per
 # tile, a step unroll of 1 or 2 four-step groups per loop iteration, and the
