@@ -263,7 +263,7 @@ __global__ __launch_bounds__(CV_MAX_THREADS) void k_cv_uniform(const KJob job, c
   const bool valid = p < P;
   const KModel& f = job.m;
   constexpr int K = NK<D, FAM>::K;
-  NormalStream ns;
+  NormalStream<> ns;
   ns.init((uint32_t)job.seed, (uint32_t)(job.seed >> 32), job.path_offset + (uint64_t)p);
   float x[D];
 #pragma unroll
@@ -303,7 +303,8 @@ __global__ __launch_bounds__(CV_MAX_THREADS) void k_cv_uniform(const KJob job, c
 // f(t_n, X_n) . dW_n and compensator g(t_n, X_n-) (t_{n+1} - t_n).  Rows run
 // in lock-step across the wavefront so the products see all 64 lanes;
 // finished lanes ride along with their results masked.
-template <int D, int FAM>
+// HELD: the normals' products held along the path (launch_cv_adapted_d).
+template <int D, int FAM, bool HELD = false>
 __global__ __launch_bounds__(CV_MAX_THREADS) void k_cv_adapted(const KJob job, const uint16_t* fw,
                                                     int32_t f_hidden, const uint16_t* gw,
                                                     int32_t g_hidden, float rate, float comp,
@@ -328,7 +329,7 @@ __global__ __launch_bounds__(CV_MAX_THREADS) void k_cv_adapted(const KJob job, c
   c.P = P;
   c.k0 = (uint32_t)job.seed;
   c.k1 = (uint32_t)(job.seed >> 32);
-  AdaptRngSrc<D, FAM> src;
+  AdaptRngSrc<D, FAM, HELD> src;
   src.init(f, c);
   const float T32 = (float)job.T;
   const int32_t max_steps = job.max_steps;
@@ -459,12 +460,25 @@ template <int D, int FAM>
 int launch_cv_adapted_d(const KJob& job, const CvLaunch& a, int64_t nchunks) {
   static const int vgprs = cv_kernel_vgprs((const void*)k_cv_adapted<D, FAM>);
   const size_t lds = (size_t)(cv_words(a.f_hidden) + cv_words(a.g_hidden)) * 2;
-  const int wpb = cv_waves_per_block(nchunks, vgprs, lds);
+  // The 1-D Merton kernel is 2-5% faster with the products held, at 161 VGPRs and
+  // 3 wavefronts per SIMD (f and g of two hidden layers, 1e5 paths x 60 steps 206
+  // against 214 us), but only while the launch fits the chip at those three (2^18
+  // paths 376 against 341); the other kernels gain nothing (2-D, f and g: 5% less).
+  const bool held = D == 1 && FAM == FAM_MERTON && nchunks <= 256 * 12;
+  const int wpb = held ? 4 : cv_waves_per_block(nchunks, vgprs, lds);
   const int64_t blocks = (nchunks + wpb - 1) / wpb;
   if (blocks <= 0 || blocks > 0x7fffffffLL) return SDEMC_ERR_ARG;
-  hipLaunchKernelGGL((k_cv_adapted<D, FAM>), dim3((unsigned)blocks), dim3(WAVE * wpb), lds,
-                     a.stream, job, a.fw, a.f_hidden, a.gw, a.g_hidden, a.rate, a.comp,
-                     a.cv_steps, a.partials, a.cflags, a.gamma, nchunks);
+#define SDEMC_CV(H)                                                                           \
+  hipLaunchKernelGGL((k_cv_adapted<D, FAM, H>), dim3((unsigned)blocks), dim3(WAVE * wpb), lds, \
+                     a.stream, job, a.fw, a.f_hidden, a.gw, a.g_hidden, a.rate, a.comp,       \
+                     a.cv_steps, a.partials, a.cflags, a.gamma, nchunks)
+  if constexpr (D == 1 && FAM == FAM_MERTON) {
+    if (held) SDEMC_CV(true);
+    else SDEMC_CV(false);
+  } else {
+    SDEMC_CV(false);
+  }
+#undef SDEMC_CV
   return hipGetLastError() == hipSuccess ? SDEMC_OK : SDEMC_ERR_LAUNCH;
 }
 

@@ -33,11 +33,11 @@ __device__ __forceinline__ void chunk_body(const KJob& job, int64_t chunk, doubl
     float x[D];
     if (GRID == SDEMC_GRID_UNIFORM) {
       if (MODE == 1 || (MODE < 0 && job.pois_mode != 0))
-        path_uniform_rng_form<D, FAM, false, U, MODE != 0, false, UF>(job, c, valid, x, st);
+        path_uniform_rng_form<D, FAM, false, U, MODE != 0, false, UF, false>(job, c, valid, x, st);
       else
-        path_uniform_rng_form<D, FAM, false, U, MODE == 1, false, UF>(job, c, valid, x, st);
+        path_uniform_rng_form<D, FAM, false, U, MODE == 1, false, UF, false>(job, c, valid, x, st);
     } else {
-      AdaptQueueSrc<D, FAM> src;
+      AdaptQueueSrc<D, FAM, false> src;
       src.init(job.m, c);
       path_adapted<D, FAM, false>(job, src, valid, p, x, ovf, st);
     }
@@ -45,10 +45,10 @@ __device__ __forceinline__ void chunk_body(const KJob& job, int64_t chunk, doubl
   } else {
     float xf[D], xc[D];
     if (GRID == SDEMC_GRID_UNIFORM) {
-      if (job.pois_mode != 0) path_uniform_rng_coupled<D, FAM, true, UF>(job, c, xf, xc);
-      else path_uniform_rng_coupled<D, FAM, false, UF>(job, c, xf, xc);
+      if (job.pois_mode != 0) path_uniform_rng_coupled<D, FAM, true, UF, false>(job, c, xf, xc);
+      else path_uniform_rng_coupled<D, FAM, false, UF, false>(job, c, xf, xc);
     } else {
-      AdaptQueueSrc<D, FAM> src;
+      AdaptQueueSrc<D, FAM, false> src;
       src.init(job.m, c);
       path_adapted_coupled<D, FAM>(job, src, valid, xf, xc, ovf);
     }

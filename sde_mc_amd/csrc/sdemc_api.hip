@@ -172,7 +172,7 @@ __global__ void k_normals(uint32_t k0, uint32_t k1, uint64_t path_offset, int64_
                           int32_t n_per_path, float* out) {
   const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= n_paths) return;
-  NormalStream ns;
+  NormalStream<> ns;
   ns.init(k0, k1, path_offset + (uint64_t)p);
   for (int32_t i = 0; i < n_per_path; ++i) out[(int64_t)i * n_paths + p] = ns.get((uint32_t)i);
 }
@@ -223,7 +223,7 @@ __global__ __launch_bounds__(256) void k_valu_probe(float* __restrict__ out, int
         acc ^= w.x ^ w.y ^ w.z ^ w.w;
       } else {
         float z[NORMALS_PER_BLOCK];
-        normals6(w, z);
+        normals6<true>(w, z);
         zacc += ((z[0] + z[1]) + (z[2] + z[3])) + (z[4] + z[5]);
       }
     }

@@ -126,16 +126,27 @@ __device__ __forceinline__ void box_muller_ua(float u, float one_plus_a, float& 
 // radius does not use, and 10 bits of word 3 (126 of the block's 128 bits).
 // z[2p] = r_p cos(2 pi a_p), z[2p + 1] = r_p sin(2 pi a_p).
 constexpr int NORMALS_PER_BLOCK = 6;
+// HAND: the angles' bits in two shifts, an and-or (1.0f is an inline constant)
+// and a bit select written out. That is an operation an angle less, 1-4% of a
+// single-level plain kernel's time, but the angles are then formed early and
+// held: 4 to 8 registers more, which the batched class kernels, the storing ones
+// and the control variates (whose normals come one row at a time, 4% slower
+// with it) do not have.
+template <bool HAND>
 __device__ __forceinline__ void normals6(const U4& w, float* z) {
   const uint32_t wp[3] = {w.x, w.y, w.z};
 #pragma unroll
   for (int p = 0; p < 3; ++p) {
-    // 1 + a as float bits: 0x3F800000 | (w_p mod 2^9) << 14 | (w3 field) << 4.
-    // Left to the compiler: written as and-or and bit-select instructions by
-    // hand, the angles were formed early and held, 4 to 8 registers more in the
-    // step loops without a gain in any (320 launch shapes: 0.4% slower on average)
-    const uint32_t lo = (((w.w >> (10 * p)) & 0x3FFu) << 4) | 0x3F800000u;
-    const uint32_t bits = ((wp[p] << 14) & 0x007FC000u) | lo;
+    // 1 + a as float bits: 0x3F800000 | (w_p mod 2^9) << 14 | (w3 field) << 4
+    uint32_t lo, bits;
+    if constexpr (HAND) {
+      const uint32_t field = p == 0 ? w.w << 4 : w.w >> (10 * p - 4);
+      asm("v_and_or_b32 %0, %1, %2, 1.0" : "=v"(lo) : "v"(field), "s"(0x3FF0u));
+      asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(bits) : "s"(0x007FC000u), "v"(wp[p] << 14), "v"(lo));
+    } else {
+      lo = (((w.w >> (10 * p)) & 0x3FFu) << 4) | 0x3F800000u;
+      bits = ((wp[p] << 14) & 0x007FC000u) | lo;
+    }
     box_muller_ua(u01_open(wp[p]), __uint_as_float(bits), z[2 * p], z[2 * p + 1]);
   }
 }
@@ -145,6 +156,7 @@ __device__ __forceinline__ void normals6(const U4& w, float* z) {
 // and one that depends on the path alone, and so is one product of the second,
 // so they are taken once per path or on the scalar unit, and a block costs 36
 // vector operations instead of 41 (philox4x32_10 bit for bit).
+template <bool HAND>
 struct BmStream {
   uint32_t k0, k1;
   uint32_t lo1;     // low word of 0xCD9E8D57 plo, xor the second round's key
@@ -183,10 +195,10 @@ struct BmStream {
     return U4{c0, c1, c2, c3};
   }
   // the six normals of block b
-  __device__ __forceinline__ void normals(uint32_t b, float* z) const { normals6(block(b), z); }
+  __device__ __forceinline__ void normals(uint32_t b, float* z) const { normals6<HAND>(block(b), z); }
 };
 
-// The same blocks, each drawn from the beginning, for kernels whose occupancy
+// The same blocks, each drawn from the beginning, for a kernel whose occupancy
 // the held products cost more than the five operations a block.
 struct BmPlain {
   uint32_t k0, k1, plo, phi;
@@ -197,11 +209,9 @@ struct BmPlain {
     phi = hi;
   }
   __device__ __forceinline__ void normals(uint32_t b, float* z) const {
-    normals6(philox4x32_10(b, STREAM_BM, plo, phi, k0, k1), z);
+    normals6<false>(philox4x32_10(b, STREAM_BM, plo, phi, k0, k1), z);
   }
 };
-template <bool HELD>
-using BmBlocks = std::conditional_t<HELD, BmStream, BmPlain>;
 
 // Steps (or adapted-grid rows) whose K normals each are drawn together as
 // whole blocks: 4 when 4K normals fill whole blocks (K = 3), else 6.
@@ -260,11 +270,11 @@ __device__ __forceinline__ float ln_unit(uint32_t w) {
 
 // Normal number i of one path (i = step * K + k): normal i mod 6 of Philox
 // block i / 6 on the Brownian stream (normals6).  The last block is cached,
-// so sequential reads cost one Philox block per 6 normals.  The control-variate
-// kernels read it beside their accumulators: with the held products the 1-D
-// Merton one took 161 VGPRs, 3 wavefronts per SIMD, instead of 128 and 4.
+// so sequential reads cost one Philox block per 6 normals.  HELD: the path's
+// products held (BmStream).
+template <bool HELD = false>
 struct NormalStream {
-  BmPlain bm;
+  std::conditional_t<HELD, BmStream<true>, BmPlain> bm;
   uint32_t blk;
   float z[NORMALS_PER_BLOCK];
   __device__ __forceinline__ void init(uint32_t key0, uint32_t key1, uint64_t path) {
@@ -1379,7 +1389,9 @@ struct CoarseAcc {
 // COUPLED: x is the fine path of an MLMC pair and xc (then non-null) its
 // coarse path, stepped every M = j.M fine steps by CoarseAcc.
 // UF: the step form the loop is compiled for (uniform_step).
-template <int D, int FAM, bool STORE, int U, bool POIS, bool COUPLED = false, int UF = UFORM_ANY>
+// HAND: the normals' angle bits (normals6).
+template <int D, int FAM, bool STORE, int U, bool POIS, bool COUPLED = false, int UF = UFORM_ANY,
+          bool HAND = true>
 __device__ void path_uniform_rng_form(const KJob& j, const PathCtx& c, bool lane_valid,
                                       float (&x)[D], const StoreCtx& st,
                                       float* xc = nullptr) {
@@ -1391,11 +1403,14 @@ __device__ void path_uniform_rng_form(const KJob& j, const PathCtx& c, bool lane
   const float sq = j.sqh;
   const uint32_t plo = (uint32_t)c.path, phi = (uint32_t)(c.path >> 32);
   constexpr bool pois = POIS;
-  // products held along the path but where registers are short: a coupled
-  // pair's general loop, and storing kernels, whose addresses take theirs (4-D
-  // Merton 71 VGPRs, 92 with them and the loop below in full groups: 7 -> 5
-  // wavefronts per SIMD, 2e5 paths x 96 steps 185 -> 219 us)
-  BmBlocks<!STORE && !(COUPLED && UF == UFORM_ANY)> bm;
+  // Storing kernels of two or more components are short of registers, their
+  // arrays' addresses taking some: no products held along the path, the angle bits
+  // left to the compiler and one loop with end tests instead of full groups and
+  // a loop for the last steps (4-D Merton 72 VGPRs instead of 92, 7 wavefronts per
+  // SIMD instead of 5: 2e5 paths x 96 steps 218 -> 185 us; 2-D, 1e4 paths 55 -> 52).
+  constexpr bool LEAN = STORE && D > 1;
+  static_assert(!LEAN || U == 1, "the lean loop takes one group a turn");
+  BmStream<HAND> bm;
   bm.init(c.k0, c.k1, plo, phi);
   // the common forms' jump coefficients: the exponential Levy's are constant,
   // the proportional ones are not (takes_common_form asks for both)
@@ -1505,7 +1520,12 @@ __device__ void path_uniform_rng_form(const KJob& j, const PathCtx& c, bool lane
     const uint32_t b0 = (uint32_t)n0 * (uint32_t)K / (uint32_t)NORMALS_PER_BLOCK;
 #pragma unroll
     for (int b = 0; b < G * K / NORMALS_PER_BLOCK; ++b)
-      bm.normals(b0 + b, &z[NORMALS_PER_BLOCK * b]);
+      // (a coupled pair's general loop is short of registers too: no products held)
+      if constexpr (LEAN || (COUPLED && UF == UFORM_ANY))
+        normals6<HAND && !LEAN>(philox4x32_10(b0 + b, STREAM_BM, plo, phi, c.k0, c.k1),
+                                &z[NORMALS_PER_BLOCK * b]);
+      else
+        bm.normals(b0 + b, &z[NORMALS_PER_BLOCK * b]);
 #pragma unroll
     for (int s = 0; s < G; ++s) {
       const int32_t n = n0 + s;
@@ -1517,12 +1537,10 @@ __device__ void path_uniform_rng_form(const KJob& j, const PathCtx& c, bool lane
         for (int i = 0; i < D; ++i) xo[i] = x[i];
         uniform_step<D, FAM, UF>(j, x, &z[s * K], fine, UF == UFORM_PROP ? uA : j.uA);
         float jsum = 0.0f;
-        // a common form's step without a jump runs straight on, the jumps laid
-        // out of line; the general form's tests its lanes in line (out of line
-        // its small launches, whose wavefronts meet a jump at most steps, take
-        // two branches more a step: 1e4 3-D Merton paths of mixed coefficients
-        // x 96 steps 52.4 us against 49.3)
-        if (!pois && (UF == UFORM_ANY ? n == hk : (bool)__builtin_expect(__any(n == hk), 0))) {
+        // rare enough (and long) to be laid out of line: steps without a jump
+        // run straight on (in line, the general form's launches without jumps
+        // take up to a third more, those with a jump at most steps 4% less)
+        if (!pois && __builtin_expect(__any(n == hk), 0)) {
           while (n == hk) {
             const float J = cq->J[qh][lane];
             if (additive) {  // fma(j1, y, j0) = j0 exactly: add_jump's bits, one operation
@@ -1656,32 +1674,26 @@ __device__ void path_uniform_rng_form(const KJob& j, const PathCtx& c, bool lane
       spill = __any(kj < wend);
     }
   };
-  // the general form of larger states and of storing kernels keeps the end
-  // tests, in one loop: without them the compiler holds more values across
-  // steps than the wavefronts pay for, and a second loop for the last steps
-  // doubles its code (1e4 2-D Merton paths x 96 steps stored 56.7 us against 51.8)
-  constexpr bool FULL = !(UF == UFORM_ANY && (STORE || D > (COUPLED ? 1 : 2)));
-  using Full = std::bool_constant<FULL>;
+  // the general form of larger states keeps the end tests: without them the
+  // compiler holds more values across steps than the wavefronts pay for
+  using Full = std::bool_constant<!(UF == UFORM_ANY && D > (COUPLED ? 1 : 2)) && !LEAN>;
   int32_t n0 = 0;
-  for (; FULL ? n0 + G * U <= N : n0 < N; n0 += G * U) {
+  for (; LEAN ? n0 < N : n0 + G * U <= N; n0 += G * U) {
     window(n0);
     if (spill) {
 #pragma unroll
-      for (int u = 0; u < U; ++u)
-        if (FULL || u == 0 || n0 + G * u < N) group(n0 + G * u, std::true_type{}, Full{});
+      for (int u = 0; u < U; ++u) group(n0 + G * u, std::true_type{}, Full{});
     } else {
 #pragma unroll
-      for (int u = 0; u < U; ++u)
-        if (FULL || u == 0 || n0 + G * u < N) group(n0 + G * u, std::false_type{}, Full{});
+      for (int u = 0; u < U; ++u) group(n0 + G * u, std::false_type{}, Full{});
     }
   }
-  if constexpr (FULL) {
-    // the last steps of a grid that is no multiple of the stride
+  // the last steps of a grid that is no multiple of the stride
+  if constexpr (!LEAN)
     for (; n0 < N; n0 += G) {
       window(n0);
       group(n0, std::true_type{}, std::false_type{});
     }
-  }
 }
 
 __host__ __device__ constexpr bool is_common_form(int form, int32_t uform, int32_t additive,
@@ -1708,11 +1720,11 @@ __host__ __device__ __forceinline__ bool takes_common_form(const KJob& j) {
 // it shares the 4-step normal blocks, the jump queue and the per-wavefront
 // jump lists; the draws, their order and the arithmetic are those of
 // path_uniform_coupled.
-template <int D, int FAM, bool POIS, int UF>
+template <int D, int FAM, bool POIS, int UF, bool HAND = true>
 __device__ __forceinline__ void path_uniform_rng_coupled(const KJob& j, const PathCtx& c,
                                                          float (&xf)[D], float (&xc)[D]) {
   const StoreCtx st{};
-  path_uniform_rng_form<D, FAM, false, 1, POIS, true, UF>(j, c, true, xf, st, xc);
+  path_uniform_rng_form<D, FAM, false, 1, POIS, true, UF, HAND>(j, c, true, xf, st, xc);
 }
 
 // Row layout of fixed increments per step: D ('diag'), D + 1 ('indep'
@@ -1946,9 +1958,9 @@ __device__ __forceinline__ bool isclose32(float tau, float t) {
 // Philox block and the arrival times accumulate in the same fp32 order as a
 // jump-by-jump clock, so the grid and the marks do not depend on when the
 // draws happen.
-template <int D, int FAM>
+template <int D, int FAM, bool HELD = false>
 struct AdaptRngSrc {
-  NormalStream ns;
+  NormalStream<HELD> ns;
   JumpClock jc;  // the last jump drawn
   uint32_t plo, phi, k0, k1;
   float tau1, J1, tau2, J2;  // tau2 < 0: no second jump drawn
@@ -2009,11 +2021,11 @@ struct AdaptRngSrc {
 // clock.  Two jump slots per lane in registers, refilled for the wavefront about
 // twice per jump, left a tenth of the jumps to be drawn by one lane alone; the
 // queue leaves almost none.
-template <int D, int FAM>
+template <int D, int FAM, bool HAND = true>
 struct AdaptQueueSrc {
   JumpClock jc;  // the last jump drawn
   uint32_t plo, phi, k0, k1, lane;
-  BmStream bm;
+  BmStream<HAND> bm;
   uint32_t head;
   ClockLds* cq;
   __device__ __forceinline__ void put(const KModel& f) {

@@ -1,6 +1,7 @@
 """Control-variate launches around the size from which workgroups of eight
-wavefronts are taken (2048 chunks of 64 paths), one and two networks, one and
-two dimensions: every path's value is the one a small launch gives it, bit for
+wavefronts are taken (2048 chunks of 64 paths) and the one up to which the 1-D
+kernel holds the normals' products (3072), one and two networks, one and two
+dimensions: every path's value is the one a small launch gives it, bit for
 bit, and the last chunk's ragged end too."""
 import pytest
 import torch
@@ -16,7 +17,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize('dim', [1, 2])
 @pytest.mark.parametrize('nets', ['f', 'g', 'f and g'])
-@pytest.mark.parametrize('chunks', [2047, 2048, 2049])
+@pytest.mark.parametrize('chunks', [2047, 2048, 3072, 3073])
 def test_values_do_not_depend_on_the_launch(dim, nets, chunks):
     dev = E.require_device()
     torch.manual_seed(dim)

@@ -28,7 +28,7 @@ def test_batched_class_kernels_do_not_spill(cls, waves):
 
 def test_control_variate_kernels_keep_their_wavefronts():
     # the 1-D Merton kernel's workgroups of eight rest on four wavefronts per SIMD
-    assert kernel_notes.waves_per_simd(KERNELS['k_cv_adapted<1, 0>']) >= 4
+    assert kernel_notes.waves_per_simd(KERNELS['k_cv_adapted<1, 0, false>']) >= 4
     for name, k in KERNELS.items():
         if name.startswith('k_cv_adapted<') or name.startswith('k_cv_uniform<'):
             assert kernel_notes.waves_per_simd(k) >= (4 if 'uniform' in name else 3), name
@@ -43,8 +43,8 @@ def test_fixed_increment_adapted_kernels_hold_no_event_state():
 @pytest.mark.parametrize('family', ['0', '1'])
 @pytest.mark.parametrize('pois', ['false', 'true'])
 def test_storing_uniform_kernels_keep_their_wavefronts(family, pois):
-    # up to 4 components, beside the addresses of three stored arrays
-    for dim, waves in ((1, 8), (2, 8), (3, 7), (4, 6)):
+    # two to four components, beside the addresses of three stored arrays
+    for dim, waves in ((2, 8), (3, 7), (4, 6)):
         k = KERNELS['k_rng<%d, %s, 0, false, true, %s, -1>' % (dim, family, pois)]
         assert k['.private_segment_fixed_size'] == 0
         assert kernel_notes.waves_per_simd(k) >= waves
