@@ -1404,13 +1404,15 @@ __device__ void path_uniform_rng_form(const KJob& j, const PathCtx& c, bool lane
   const uint32_t plo = (uint32_t)c.path, phi = (uint32_t)(c.path >> 32);
   constexpr bool pois = POIS;
   // Storing kernels of two or more components are short of registers, their
-  // arrays' addresses taking some: no products held along the path, the angle bits
-  // left to the compiler and one loop with end tests instead of full groups and
-  // a loop for the last steps (4-D Merton 72 VGPRs instead of 92, 7 wavefronts per
-  // SIMD instead of 5: 2e5 paths x 96 steps 218 -> 185 us; 2-D, 1e4 paths 55 -> 52).
+  // arrays' addresses taking some: the angle bits are left to the compiler and one
+  // loop with end tests stands for full groups and a loop for the last steps (4-D
+  // 73-90 VGPRs instead of 92-101, and the per-step counts' 20-36 spilled bytes a
+  // lane gone: 1e4 paths x 96 steps, Merton 83.5 -> 80.0 us, Levy 122.4 -> 115.0; 2e5
+  // paths, which the writes bound, 217 and 278 either way).  Without the products
+  // held along the path too (72 VGPRs), launches without jumps took 3% more.
   constexpr bool LEAN = STORE && D > 1;
   static_assert(!LEAN || U == 1, "the lean loop takes one group a turn");
-  BmStream<HAND> bm;
+  BmStream<HAND && !LEAN> bm;
   bm.init(c.k0, c.k1, plo, phi);
   // the common forms' jump coefficients: the exponential Levy's are constant,
   // the proportional ones are not (takes_common_form asks for both)
@@ -1520,10 +1522,10 @@ __device__ void path_uniform_rng_form(const KJob& j, const PathCtx& c, bool lane
     const uint32_t b0 = (uint32_t)n0 * (uint32_t)K / (uint32_t)NORMALS_PER_BLOCK;
 #pragma unroll
     for (int b = 0; b < G * K / NORMALS_PER_BLOCK; ++b)
-      // (a coupled pair's general loop is short of registers too: no products held)
-      if constexpr (LEAN || (COUPLED && UF == UFORM_ANY))
-        normals6<HAND && !LEAN>(philox4x32_10(b0 + b, STREAM_BM, plo, phi, c.k0, c.k1),
-                                &z[NORMALS_PER_BLOCK * b]);
+      // (a coupled pair's general loop is short of registers: no products held)
+      if constexpr (COUPLED && UF == UFORM_ANY)
+        normals6<HAND>(philox4x32_10(b0 + b, STREAM_BM, plo, phi, c.k0, c.k1),
+                       &z[NORMALS_PER_BLOCK * b]);
       else
         bm.normals(b0 + b, &z[NORMALS_PER_BLOCK * b]);
 #pragma unroll
